@@ -1,0 +1,157 @@
+"""Plane tiles on the GPU: every committed trace with each tile forced, under
+the kernel-boundary parity of tests/test_gpu_parity.py; contractions at the
+edges of tiles, groups and K splits against float64; operands that do not
+split into bf16 planes (infinities, NaN, the largest and the smallest
+values); and the routes by size.
+
+Bounds: a sum of K products in any order of f32 additions is within
+K * 2^-24 of the sum of the products' magnitudes; the products left out of
+the split add less than 2^-24 of it. f16 results are rounded once more
+(2^-11, and half the smallest f16 step)."""
+import os
+
+import numpy as np
+import pytest
+
+from tests import contractions as ct
+from tests import tracetools as tt
+from tests.test_gpu_dense import dense_tolerance
+from tests.test_gpu_parity import _oracle, kernel_parity
+from tinyhvm_amd import _lib, abi
+
+pytestmark = pytest.mark.gpu
+F32, F16 = abi.DTYPE_F32, abi.DTYPE_F16
+KNOBS = ("THVM_HIP_DENSE_FORCE", "THVM_HIP_DENSE_SPLITS", "THVM_HIP_DENSE_TILE")
+
+
+def _init(force, splits, tile):
+    saved = {k: os.environ.get(k) for k in KNOBS}
+    os.environ.update(zip(KNOBS, (force, splits, tile)))
+    L = _lib.lib()
+    L.thvm_hip_shutdown()
+    assert L.thvm_hip_init() == 0
+    return L, saved
+
+
+def _fini(L, saved):
+    L.thvm_hip_shutdown()
+    for k, v in saved.items():
+        if v is None:
+            os.environ.pop(k, None)
+        else:
+            os.environ[k] = v
+
+
+# (split-K, tile): 12 and 13 128x128 (two LDS stages, one), 14 and 15 128x64, 16 and 17 64x64; 0 by size
+@pytest.fixture(scope="module", params=[("1", "12"), ("3", "13"), ("2", "14"), ("1", "15"), ("3", "16"), ("1", "17"), ("0", "0")],
+                ids=["128x128d", "128x128-split3", "128x64d-split2", "128x64", "64x64d-split3", "64x64", "by-size"])
+def hip(request):
+    L, saved = _init("1" if request.param[1] != "0" else "0", *request.param)
+    yield L
+    _fini(L, saved)
+
+
+@pytest.mark.parametrize("path", tt.fixtures(), ids=lambda p: p.split("/")[-1])
+def test_trace_parity(hip, path):
+    kr, e2e = kernel_parity(hip.thvm_hip_backend(), hip.thvm_hip_buf_read, hip.thvm_hip_synchronize, _oracle(), path,
+                            tol_fn=dense_tolerance)
+    assert not [r for r in kr if not r[1]], kr
+    assert not [r for r in e2e if not r[1]], e2e
+
+
+def _dispatch(L, k, a, b, n_out, out_dt):
+    import ctypes as C
+    ids = []
+    try:
+        for x in (a, b):
+            i = L.thvm_hip_buf_alloc(x.nbytes)
+            L.thvm_hip_buf_write(i, x.ctypes.data_as(C.c_void_p), x.nbytes)
+            ids.append(i)
+        out = np.full(n_out, np.nan, np.float16 if out_dt == F16 else np.float32)
+        o = L.thvm_hip_buf_alloc(out.nbytes)
+        L.thvm_hip_buf_write(o, out.ctypes.data_as(C.c_void_p), out.nbytes)
+        ids.append(o)
+        L.thvm_hip_dispatch_uop_kernel(o, (C.c_uint32 * 2)(*ids[:2]), 2, C.byref(k), 0)
+        L.thvm_hip_buf_read(o, out.ctypes.data_as(C.c_void_p), out.nbytes)
+        assert L.thvm_hip_synchronize() == 0
+        return out
+    finally:
+        for i in ids:
+            L.thvm_hip_buf_free(i)
+
+
+def _check(L, kind, k, a, b, kk, dt):
+    with np.errstate(all="ignore"):
+        want, mag = ct.reference(kind, a, b)
+    got = _dispatch(L, k, a, b, want.size, dt).astype(np.float64).reshape(want.shape)
+    with np.errstate(all="ignore"):
+        ref = want.astype(np.float16 if dt == F16 else np.float32).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(got[inf], ref[inf])
+    ok = np.isfinite(ref)
+    bound = (kk + 2) * 2.0 ** -24 * mag[ok] + 2.0 ** -149
+    if dt == F16:
+        bound = bound + np.abs(want[ok]) * 2.0 ** -11 + 2.0 ** -25
+    worst = np.max(np.abs(got[ok] - want[ok]) / bound) if ok.any() else 0.0
+    assert worst <= 1.0, worst
+
+
+# edges of tiles (64, 128), of groups (4, 8), of stages (32, 64), and of pairs of rows
+SIZES = [(64, 64, 64), (128, 96, 128), (65, 33, 63), (129, 771, 130), (63, 4, 17), (16, 257, 16), (200, 130, 72), (17, 8, 300)]
+
+
+@pytest.mark.parametrize("dt", [F32, F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("m,k,n", SIZES, ids=lambda v: str(v))
+@pytest.mark.parametrize("kind", ["nn", "nt", "tn"])
+def test_matmul_edges(hip, kind, m, k, n, dt):
+    prog, sa, sb = ct.matmul(kind, m, k, n, dt)
+    rng = np.random.default_rng(m * 7 + k * 3 + n)
+    f = np.float16 if dt == F16 else np.float32
+    _check(hip, kind, prog, rng.uniform(-1, 1, sa).astype(f), rng.uniform(-1, 1, sb).astype(f), k, dt)
+
+
+@pytest.mark.parametrize("shape", [(3, 8, 20, 7, 9, 3), (2, 33, 17, 11, 13, 5), (5, 16, 24, 10, 10, 1), (1, 4, 70, 12, 16, 3)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("kind", ["cf", "dw"])
+def test_convolution_edges(hip, kind, shape):
+    prog, sa, sb = ct.conv(kind, *shape)
+    rng = np.random.default_rng(sum(shape))
+    b, ci, _co, h, w, ks = shape
+    kk = ci * ks * ks if kind == "cf" else b * h * w
+    _check(hip, kind, prog, rng.standard_normal(sa).astype(np.float32), rng.standard_normal(sb).astype(np.float32), kk, F32)
+
+
+@pytest.mark.parametrize("what", ["inf", "nan", "huge", "tiny", "subnormal"])
+def test_operands_that_do_not_split(hip, what):
+    """One row, or one element, that has no exact bf16 planes; the tile it is
+    in keeps the f32 instruction's result, and its neighbours theirs."""
+    m, k, n = 200, 260, 150
+    prog, sa, sb = ct.matmul("nn", m, k, n)
+    rng = np.random.default_rng(5)
+    a, b = rng.uniform(-1, 1, sa).astype(np.float32), rng.uniform(-1, 1, sb).astype(np.float32)
+    if what == "inf":
+        a[3, 7], b[200, 100] = np.inf, -np.inf
+        a[150, 200] = 0.0                    # 0 * -inf is NaN
+    elif what == "nan":
+        a[70, 1] = np.nan
+    elif what == "huge":
+        a[5, 5] = a[5, 9] = np.float32(3.4028235e38)     # rounds past the bf16 range
+        b[5, :], b[9, :] = 0.5, 0.25
+    elif what == "tiny":
+        a[:64] *= np.float32(2.0 ** -119)
+        b *= np.float32(2.0 ** 100)
+    else:
+        a[10] = rng.integers(1, 1000, k).astype(np.float32) * np.float32(1e-45)
+        b *= np.float32(2.0 ** 110)
+    _check(hip, "nn", prog, a, b, k, F32)
+
+
+def test_f16_subnormals_and_infinities(hip):
+    prog, sa, sb = ct.matmul("nt", 70, 130, 66, F16)
+    rng = np.random.default_rng(6)
+    a, b = rng.uniform(-1, 1, sa).astype(np.float16), rng.uniform(-1, 1, sb).astype(np.float16)
+    a[3] = (rng.integers(1, 1000, 130) * 2.0 ** -24).astype(np.float16)
+    b[5] *= np.float16(512)
+    a[40, 7], b[9, 20] = np.inf, np.nan
+    _check(hip, "nt", prog, a, b, 130, F16)

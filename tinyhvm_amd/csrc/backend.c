@@ -1052,7 +1052,8 @@ static void read_dense_env(void) {
     if (hipb.gemm_depth > 2) hipb.gemm_depth = 0;
     e = getenv("THVM_HIP_DENSE_TILE");
     hipb.dense_tile = e ? (u32)atoi(e) : 0;
-    if (hipb.dense_tile > 11) hipb.dense_tile = 0;
+    if (hipb.dense_tile > 17) hipb.dense_tile = 0;
+    hipb.dense_noplanes = env_flag("THVM_HIP_DENSE_NOPLANES");
 }
 
 u32 hipb_resident_waves(void) { return hipb.resident_waves ? hipb.resident_waves : 256u * SINGLE_PASS_WAVES_PER_CU; }

@@ -316,7 +316,9 @@ typedef struct {
     u32 gm, gn;
     const char *tag;
     int direct;    /* no LDS: 1 = each wave owns one 32x32 block and loads its MFMA operands
-                      itself; 2 = skinny (see CFG_SKINNY) */
+                      itself; 2 = skinny (see CFG_SKINNY); 3 = outer product; 4 = wave tile;
+                      5 = plane tile */
+    u32 nbuf;      /* plane tile: LDS stages (2: the next stage is split and stored during the math) */
 } TileCfg;
 
 /* bk: K per LDS stage (32 halves the barriers per K of 16; measured 2-3%
@@ -366,6 +368,17 @@ static const TileCfg CFG_SKINNY = {64, 16, 1, 1, 1, 1, 1, "skinny", 2};
  * across the wavefront's lanes by shuffles, adds the four waves in order, and
  * the chunks' partials go through the split-K sum. Both sides separable. */
 static const TileCfg CFG_RED = {1, 1, 1, 1, 1, 1, 1, "outer", 3};
+/* Plane tiles (emit_plane_kernel): both operands staged in LDS as 16-bit
+ * planes with k contiguous and multiplied by the 16-bit matrix instructions. */
+static const TileCfg CFG_PLANE[] = {
+    {128, 128, 32, 2, 1, 2, 4, "plane128x128d", 5, 2},
+    {128, 128, 32, 2, 2, 2, 2, "plane128x128", 5, 1},
+    {128, 64, 32, 2, 1, 2, 2, "plane128x64d", 5, 2},
+    {128, 64, 32, 2, 1, 2, 2, "plane128x64", 5, 1},
+    {64, 64, 32, 1, 1, 2, 2, "plane64x64d", 5, 2},
+    {64, 64, 32, 1, 1, 2, 2, "plane64x64", 5, 1},
+};
+#define N_PLANE ((u32)(sizeof CFG_PLANE / sizeof CFG_PLANE[0]))
 #define RED_MAX_MN 4096
 #define RED_MIN_K 8192
 #define RED_MAX_ACC 96        /* MG * N */
@@ -401,9 +414,46 @@ typedef struct {
     int vec[2];                  /* a linear side loaded 4 contiguous, 16-byte aligned elements per lane */
 } KPerm;
 
+/* Why plane tiles, measured against the direct kernel they replace (one
+ * MI355X, a contraction alone): 1031x1501 over 771 86.7 -> 30.7 us, 1031x771
+ * over 1501 153 -> 29 us, 2048^3 in f16 445 -> 31 us (38 -> 560 TFLOP/s); the
+ * convolution of 128 channels over [32,128,28,28] 126 -> 50 us (58 -> 148
+ * TFLOP/s) forward, 376 -> 47 us for its weight gradient. A full grid of
+ * 128x128 tiles runs at 190 TFLOP/s (six bf16 products each: 1140, where
+ * hipBLASLt's largest bf16 product reaches 1209 on the same card): bound by
+ * the matrix pipes' power, then by the vector instructions of the split (6
+ * an element and stage, issued between the matrix ones).
+ *
+ * K of a plane tile: the reduce index is walked in groups of G consecutive
+ * values of one digit (the inner one, extent E); a group is what one lane
+ * loads at once. A run of E values holds Q = ceil(E / G) groups: the last one
+ * starts at E - G, so that no load leaves the run, and its first Q * G - E
+ * elements, which the group before it covers, enter as 0 on both sides. Any
+ * K with a digit of at least G values splits this way. */
+#define PLANE_GROUPS 8u          /* groups per LDS stage */
+#define PLANE_MIN_WORK (1ull << 21)
+#define PLANE_MIN_SIDE 16u       /* outputs per side: at most three quarters of a 64-wide tile empty */
+#define PLANE_PACK_MIN_TILES 8u  /* row tiles that read a packed B side */
+typedef struct {
+    u32 planes;                  /* 0: no plane tile; 1: f16 operands as they are; 3: f32 operands, each
+                                    split into three bf16 planes */
+    u32 G, E, Q, NG;             /* NG = K / E * Q groups in all */
+    u32 stages, st_chunk;        /* stages in all, and per K split */
+    u32 ndig;                    /* outer digits, fastest first */
+    u32 oext[KP_MAX];
+    u32 ocoef[2][KP_MAX];
+    u32 icoef[2];                /* per side: coefficient of the inner digit */
+    u64 maxidx[2];               /* largest element index a side can form */
+    u32 buf[2];                  /* the buffer each side loads (1 + leaf) */
+    int kmajor[2];               /* lanes along k (by groups), else along the tile's rows */
+    int vec[2];                  /* k-major: a group in one 16-byte load; row-major f16: two rows a load */
+    u32 icoef_q;                 /* the B side's own inner coefficient where it is packed (icoef is then 1) */
+} KPlane;
+
 typedef struct {
     char name[48];
     TileCfg cfg;
+    KPlane pn;
     u32 pad_a, pad_b;      /* LDS row padding (floats) of the A and B stages */
     u32 splits;
     u32 splits_want;       /* split count asked for; splits is what the K chunks give */
@@ -416,6 +466,7 @@ typedef struct {
                               run along m in the epilogue (coalesced stores) */
     int pack;              /* the B side is first copied into a K x N row-major buffer in the
                               reordered k order (a small operand with scattered loads) */
+    u64 pk_elems;          /* ... of this many floats */
     KPerm kpo;             /* the K-reordered plan before packing (the pack kernel's loads) */
     u32 ske;               /* skinny: K walked in blocks of ske (a digit boundary of both sides'
                               k offsets), whose in-block offsets are constants; 0 = per k */
@@ -447,12 +498,15 @@ static u32 dense_cus(void) { return hipb.n_cu ? hipb.n_cu : 256u; }
 
 /* lanes of an LDS tile's workgroup: one wave per gm x gn position (the
  * kernels without LDS tiles plan their loaders against GEMM_THREADS) */
-static u32 lds_threads(const TileCfg *cf) { return cf->direct ? GEMM_THREADS : 64u * cf->gm * cf->gn; }
+static u32 lds_threads(const TileCfg *cf) {
+    return cf->direct && cf->direct != 5 ? GEMM_THREADS : 64u * cf->gm * cf->gn;
+}
 
 /* workgroup size of a plan's main kernel */
 static u32 dense_threads(const GemmPlan *pl) {
     if (pl->cfg.direct == 4) return 64u * (pl->tail_s ? pl->tail_s : 1u);
-    return pl->cfg.direct == 3 ? GEMM_THREADS : pl->cfg.direct ? 64u * pl->nw : lds_threads(&pl->cfg);
+    if (pl->cfg.direct == 3) return GEMM_THREADS;
+    return pl->cfg.direct && pl->cfg.direct != 5 ? 64u * pl->nw : lds_threads(&pl->cfg);
 }
 
 /* wave tile: k-pairs of fragments in flight (a divisor of the K-pair count) */
@@ -1292,13 +1346,337 @@ static void emit_kperm_loaders(DSB *s, const Contraction *ct, const GemmPlan *pl
     }
 }
 
+/* Element offset of reduce group g on one side (see KPlane). */
+static void emit_kgroup_fn(DSB *s, const KPlane *pn, int side, u32 icoef, const char *name) {
+    dsb_put(s, "__device__ __forceinline__ u32 %s(u32 g) {\n", name);
+    if (pn->NG == pn->Q) dsb_put(s, "  const u32 j = g * %uu;\n", pn->G);
+    else dsb_put(s, "  u32 o = g / %uu;\n  const u32 j = (g %% %uu) * %uu;\n", pn->Q, pn->Q, pn->G);
+    if (pn->E % pn->G)
+        dsb_put(s, "  u32 u = (j < %uu ? j : %uu) * %uu;\n", pn->E - pn->G, pn->E - pn->G, icoef);
+    else dsb_put(s, "  u32 u = j * %uu;\n", icoef);
+    for (u32 t = 0; t < pn->ndig && pn->NG != pn->Q; t++) {
+        if (t + 1 < pn->ndig)
+            dsb_put(s, "  u += (o %% %uu) * %uu; o /= %uu;\n", pn->oext[t], pn->ocoef[side][t], pn->oext[t]);
+        else
+            dsb_put(s, "  u += o * %uu;\n", pn->ocoef[side][t]);
+    }
+    dsb_put(s, "  return u;\n}\n");
+}
+
+/* One side's loader and LDS store of a plane tile. An item of a lane's work
+ * is one group of one row (two rows of a paired row-major f16 side); r<x>[e]
+ * holds item e's raw words, o<X>[] the byte offsets of the rows it loads. */
+static void emit_plane_side(DSB *s, const Contraction *ct, const GemmPlan *pl, int side) {
+    const KPlane *pn = &pl->pn;
+    const TileCfg *cf = &pl->cfg;
+    const char X = side ? 'B' : 'A', r = side ? 'b' : 'a', S = side ? 'q' : 'p';
+    const u32 bx = side ? cf->bn : cf->bm, T = lds_threads(cf), lim = side ? ct->N : ct->M;
+    const int f16 = pn->planes == 1, kmaj = pn->kmajor[side], vec = pn->vec[side];
+    const u32 es = f16 ? 2u : 4u, G = pn->G, ic = pn->icoef[side] * es;
+    const u32 rpi = f16 && !kmaj && vec ? 2u : 1u;            /* rows per item */
+    const u32 lrow = bx / rpi;                                /* row-major: lanes side by side on one group */
+    const u32 items = lrow * PLANE_GROUPS / T, nrow = kmaj ? items : 1u;
+    const int mask = pn->E % G || pn->NG % PLANE_GROUPS;
+    const int uni = !kmaj && lrow % 64u == 0;                 /* a group's offset is one for the wave (scalar) */
+    char grp[96], off[32];
+    if (kmaj) snprintf(grp, sizeof grp, "tid %% %uu", PLANE_GROUPS);
+    else if (uni) snprintf(grp, sizeof grp, "__builtin_amdgcn_readfirstlane(tid / %uu) + e * %uu", lrow, T / lrow);
+    else snprintf(grp, sizeof grp, "tid / %uu + e * %uu", lrow, T / lrow);
+    snprintf(off, sizeof off, kmaj ? "o%c[e] + go" : uni ? "o%c[0]" : "o%c[0] + go", X);
+    if (side && pl->pack)
+        dsb_put(s, "  const __amdgpu_buffer_rsrc_t dB = __builtin_amdgcn_make_buffer_rsrc((void*)pk, (short)0, (int)%lluu, 0x00020000);\n",
+                (unsigned long long)pl->pk_elems * 4u);
+    else
+        dsb_put(s, "  const __amdgpu_buffer_rsrc_t d%c = __builtin_amdgcn_make_buffer_rsrc((void*)p%u, (short)0,\n"
+                   "      (int)((unsigned long long)c%u * %uull < 0xFFFFFFFFull ? c%u * %uu : 0xFFFFFFFFu), 0x00020000);\n",
+                X, pn->buf[side], pn->buf[side], es, pn->buf[side], es);
+    char ref[40];
+    snprintf(ref, sizeof ref, "u32 (&r%c)[%u][%u]", r, items, 4u * rpi);
+    dsb_put(s, "  u32 o%c[%u], r%c0[%u][%u];\n", X, nrow, r, items, 4u * rpi);
+    if (cf->nbuf == 2) dsb_put(s, "  u32 r%c1[%u][%u];\n", r, items, 4u * rpi);
+    dsb_put(s, "  #pragma unroll\n  for (u32 e = 0; e < %uu; e++) {\n", nrow);
+    if (kmaj)
+        dsb_put(s, "    const u32 x = %s + tid / %uu + e * %uu;\n", side ? "n0" : "m0", PLANE_GROUPS, T / PLANE_GROUPS);
+    else
+        dsb_put(s, "    const u32 x = %s + (tid %% %uu) * %uu;\n", side ? "n0" : "m0", lrow, rpi);
+    /* rows past the end are clamped: their products are never stored */
+    dsb_put(s, "    o%c[e] = row_%c(x < %uu ? x : %uu) * %uu;\n  }\n", X, S, lim, lim - rpi, es);
+    dsb_put(s, "  auto load%c = [&](u32 st, %s) {\n    #pragma unroll\n    for (u32 e = 0; e < %uu; e++) {\n"
+               "      u32 g = st * %uu + %s;\n", X, ref, items, PLANE_GROUPS, grp);
+    if (pn->NG % PLANE_GROUPS) dsb_put(s, "      g = g < %uu ? g : %uu;\n", pn->NG, pn->NG - 1);
+    dsb_put(s, "      const u32 go = kg_%c(g) * %uu;\n", S, es);
+    if (kmaj && vec)
+        dsb_put(s, "      const u4_ v = __builtin_amdgcn_raw_buffer_load_b128(d%c, (int)(%s), 0, 0);\n"
+                   "      r%c[e][0] = v.x; r%c[e][1] = v.y; r%c[e][2] = v.z; r%c[e][3] = v.w;\n", X, off, r, r, r, r);
+    else if (!f16 || rpi == 2u)
+        dsb_put(s, "      #pragma unroll\n      for (u32 j = 0; j < %uu; j++)\n"
+                   "        r%c[e][j] = __builtin_amdgcn_raw_buffer_load_b32(d%c, (int)(%s), (int)(%sj * %uu), 0);\n",
+                G, r, X, off, uni ? "go + " : "", ic);
+    else
+        dsb_put(s, "      #pragma unroll\n      for (u32 j = 0; j < 4u; j++) {\n"
+                   "        const u32 l_ = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(d%c, (int)(%s), (int)(%s2u * j * %uu), 0);\n"
+                   "        const u32 h_ = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(d%c, (int)(%s), (int)(%s(2u * j + 1u) * %uu), 0);\n"
+                   "        r%c[e][j] = l_ | (h_ << 16);\n      }\n",
+                X, off, uni ? "go + " : "", ic, X, off, uni ? "go + " : "", ic, r);
+    dsb_put(s, "    }\n  };\n"
+               "  auto store%c = [&](u32 buf, u32 st, const %s) {\n    #pragma unroll\n    for (u32 e = 0; e < %uu; e++) {\n"
+               "      const u32 gi = %s;\n", X, ref, items, grp);
+    if (kmaj) dsb_put(s, "      const u32 at = (tid / %uu + e * %uu) * LD + gi * %uu;\n", PLANE_GROUPS, T / PLANE_GROUPS, G);
+    else dsb_put(s, "      const u32 at = (tid %% %uu) * (%uu * LD) + gi * %uu;\n", lrow, rpi, G);
+    if (mask) dsb_put(s, "      const u32 z = kz(st * %uu + gi);\n", PLANE_GROUPS);
+    if (pn->planes == 3) {
+        for (u32 j = 0; j < 4; j++)
+            if (mask) dsb_put(s, "      const float x%u = %uu >= z ? __uint_as_float(r%c[e][%u]) : 0.0f;\n", j, j, r, j);
+            else dsb_put(s, "      const float x%u = __uint_as_float(r%c[e][%u]);\n", j, r, j);
+        dsb_put(s, "      u2_ h, m, l;\n"
+                   "      { u32 a, b, c; split2(x0, x1, a, b, c, bad); h.x = a; m.x = b; l.x = c;\n"
+                   "        split2(x2, x3, a, b, c, bad); h.y = a; m.y = b; l.y = c; }\n"
+                   "      *(u2_*)&%cs[buf][0][at] = h; *(u2_*)&%cs[buf][1][at] = m; *(u2_*)&%cs[buf][2][at] = l;\n", X, X, X);
+    } else {
+        for (u32 q = 0; q < rpi; q++) {
+            dsb_put(s, "      {\n        u4_ w;\n");
+            for (u32 j = 0; j < 4; j++) {
+                char v[96];
+                if (rpi == 1) snprintf(v, sizeof v, "r%c[e][%u]", r, j);
+                else if (q == 0)
+                    snprintf(v, sizeof v, "(r%c[e][%u] & 0xFFFFu) | (r%c[e][%u] << 16)", r, 2 * j, r, 2 * j + 1);
+                else
+                    snprintf(v, sizeof v, "(r%c[e][%u] >> 16) | (r%c[e][%u] & 0xFFFF0000u)", r, 2 * j, r, 2 * j + 1);
+                if (mask)
+                    dsb_put(s, "        w[%u] = (%s) & ((%uu >= z ? 0xFFFFu : 0u) | (%uu >= z ? 0xFFFF0000u : 0u));\n", j, v,
+                            2 * j, 2 * j + 1);
+                else
+                    dsb_put(s, "        w[%u] = %s;\n", j, v);
+            }
+            dsb_put(s, "        *(u4_*)&%cs[buf][0][at + %uu * LD] = w;\n      }\n", X, q);
+        }
+    }
+    dsb_put(s, "    }\n  };\n");
+}
+
+/* The plane-tile kernel (CFG_PLANE): both operands go through LDS as 16-bit
+ * planes, [plane][row][k], and the tile is multiplied with the 16-bit matrix
+ * instructions, which run 16 times the rate of v_mfma_f32_32x32x2f32.
+ *
+ * f16 operands are one plane: a product of two f16 values is exact in f32,
+ * and the instruction adds in f32, so this is the same sum as that of the
+ * widened operands, in another order.
+ *
+ * f32 operands are three bf16 planes: x = h + m + l exactly, each the
+ * rounding to nearest of what the ones before it leave (8 significant bits
+ * each, 24 in all). Of the nine products the six of weight 2^-18 and more are
+ * kept, smallest first: hl, lh, mm, mh, hm, hh. Those left out are below
+ * 2^-25 of the product and of either sign, less than the rounding of an f32
+ * accumulation step, of which there are fewer (one per 16 k and product,
+ * against one per 2 k): against 64-bit sums the error measured 0.65-0.8 of
+ * the f32 instruction's at K = 32 to 4096, on U(-1, 1) and on U(0, 1).
+ *
+ * The products but hh go into accumulators of their own (`cor`), so that the
+ * large sums are rounded once per 16 k.
+ *
+ * The split is not exact for infinities, NaNs and values that round past the
+ * bf16 range, which leave a non-finite value in every sum they enter, nor for
+ * values below about 2^-110, whose last bits are under the bf16 range: the
+ * rest they leave for the third plane does not fit its upper 16 bits (`bad`
+ * collects them). A workgroup that sees either computes its tile again with
+ * the f32 instruction from the operands themselves.
+ *
+ * One stage (PLANE_GROUPS groups of k) of LDS per workgroup; the next
+ * stage's global loads are in flight across the matrix instructions. */
+static void emit_plane_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl) {
+    const KPlane *pn = &pl->pn;
+    const TileCfg *cf = &pl->cfg;
+    const u32 WM = cf->wm_b, WN = cf->wn_b;
+    const int f16 = pn->planes == 1;
+    const char *op = f16 ? "__builtin_amdgcn_mfma_f32_32x32x16_f16" : "__builtin_amdgcn_mfma_f32_32x32x16_bf16";
+    dsb_put(s,
+            "  constexpr u32 BM = %uu, BN = %uu, BK = %uu, LD = BK + 8u, PL = %uu;\n"
+            "  constexpr u32 M = %uu, N = %uu, TM = %uu, TN = %uu, TILES = %uu, SPLITS = %uu;\n"
+            "  constexpr u32 WM = %uu, WN = %uu, GN = %uu, NST = %uu, STC = %uu;\n"
+            "  constexpr u32 KG = %uu, NGRP = %uu, ICP = %uu, ICQ = %uu;\n"
+            "  __shared__ __attribute__((aligned(16))) unsigned short As[%u][PL][BM * LD], Bs[%u][PL][BN * LD];\n"
+            "  const u32 tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;\n"
+            "  u32 bid = blockIdx.x, spl = blockIdx.y;\n"
+            "  /* the tile order of the LDS tiles: a compact block of tiles, or every\n"
+            "   * tile of a split, per XCD */\n"
+            "  if (SPLITS > 1u && SPLITS %% 8u == 0u && TILES %% 8u != 0u) {\n"
+            "    const u32 lin = blockIdx.y * TILES + blockIdx.x, j = lin / 8u;\n"
+            "    spl = (j / TILES) * 8u + lin %% 8u; bid = j %% TILES; }\n"
+            "  u32 tile = bid;\n"
+            "  if (TILES %% 8u == 0u) tile = (bid %% 8u) * (TILES / 8u) + bid / 8u;\n"
+            "  u32 tm, tn;\n"
+            "  { const u32 G = 8u; const u32 grp = tile / (G * TN), first = grp * G;\n"
+            "    const u32 gsz = (TM - first) < G ? (TM - first) : G;\n"
+            "    tm = first + (tile %% (G * TN)) %% gsz; tn = (tile %% (G * TN)) / gsz; }\n"
+            "  const u32 m0 = tm * BM, n0 = tn * BN;\n"
+            "  const u32 wm = (wave / GN) * (WM * 32u), wn = (wave %% GN) * (WN * 32u);\n"
+            "  const u32 st0 = spl * STC, st1 = st0 + STC < NST ? st0 + STC : NST;\n"
+            "  f32x16 acc[WM * WN];\n"
+            "  #pragma unroll\n  for (u32 b = 0; b < WM * WN; b++) acc[b] = (f32x16){0};\n%s",
+            cf->bm, cf->bn, pn->G * PLANE_GROUPS, pn->planes, ct->M, ct->N, pl->tiles_m, pl->tiles_n,
+            pl->tiles_m * pl->tiles_n, pl->splits, WM, WN, cf->gn, pn->stages, pn->st_chunk, pn->G, pn->NG, pn->icoef[0], pn->icoef[1],
+            cf->nbuf, cf->nbuf,
+            f16 ? "" : "  f32x16 cor[WM * WN];\n"
+                       "  #pragma unroll\n  for (u32 b = 0; b < WM * WN; b++) cor[b] = (f32x16){0};\n"
+                       "  u32 bad = 0u;\n");
+    for (int side = 0; side < 2; side++) emit_plane_side(s, ct, pl, side);
+    dsb_put(s,
+            "  auto math = [&](u32 buf) {\n"
+            "    #pragma unroll\n"
+            "    for (u32 kk = 0; kk < BK; kk += 16u) {\n"
+            "      const u32 ko = kk + (lane >> 5) * 8u;\n"
+            "      pl8_ a[PL][WM], b[PL][WN];\n"
+            "      #pragma unroll\n"
+            "      for (u32 p = 0; p < PL; p++) {\n"
+            "        #pragma unroll\n"
+            "        for (u32 i = 0; i < WM; i++) a[p][i] = *(const pl8_*)&As[buf][p][(wm + i * 32u + (lane & 31u)) * LD + ko];\n"
+            "        #pragma unroll\n"
+            "        for (u32 j = 0; j < WN; j++) b[p][j] = *(const pl8_*)&Bs[buf][p][(wn + j * 32u + (lane & 31u)) * LD + ko];\n"
+            "      }\n");
+    static const u32 pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+    for (u32 t = f16 ? 5u : 0u; t < 6; t++)
+        dsb_put(s,
+                "      #pragma unroll\n      for (u32 i = 0; i < WM; i++)\n        #pragma unroll\n"
+                "        for (u32 j = 0; j < WN; j++) %s[i * WN + j] = %s(%s, %s, %s[i * WN + j], 0, 0, 0);\n",
+                t < 5u ? "cor" : "acc", op, pl->swap ? (pb[t] == 0 ? "b[0][j]" : pb[t] == 1 ? "b[1][j]" : "b[2][j]")
+                             : (pa[t] == 0 ? "a[0][i]" : pa[t] == 1 ? "a[1][i]" : "a[2][i]"),
+                pl->swap ? (pa[t] == 0 ? "a[0][i]" : pa[t] == 1 ? "a[1][i]" : "a[2][i]")
+                         : (pb[t] == 0 ? "b[0][j]" : pb[t] == 1 ? "b[1][j]" : "b[2][j]"),
+                t < 5u ? "cor" : "acc");
+    dsb_put(s, "    }\n  };\n");
+    if (cf->nbuf == 2)
+        /* two LDS stages: while stage st is multiplied the next one, whose
+         * loads were issued a stage before, is split and stored, and the one
+         * after it loaded (past the end: the last stage again, never used) */
+        dsb_put(s,
+                "  auto step = [&](u32 st, u32 cur, auto& ra, auto& rb, auto& na, auto& nb) {\n"
+                "    const u32 s1 = st + 1u < st1 ? st + 1u : st1 - 1u, s2 = st + 2u < st1 ? st + 2u : st1 - 1u;\n"
+                "    loadA(s2, na); loadB(s2, nb);\n"
+                "    math(cur);\n"
+                "    storeA(cur ^ 1u, s1, ra); storeB(cur ^ 1u, s1, rb);\n"
+                "    __syncthreads();\n"
+                "  };\n"
+                "  if (st0 < st1) {\n"
+                "    const u32 s1 = st0 + 1u < st1 ? st0 + 1u : st0;\n"
+                "    loadA(st0, ra0); loadB(st0, rb0); loadA(s1, ra1); loadB(s1, rb1);\n"
+                "    storeA(0u, st0, ra0); storeB(0u, st0, rb0);\n"
+                "    __syncthreads();\n"
+                "    for (u32 st = st0; st < st1; st += 2u) {\n"
+                "      step(st, 0u, ra1, rb1, ra0, rb0);\n"
+                "      if (st + 1u < st1) step(st + 1u, 1u, ra0, rb0, ra1, rb1);\n"
+                "    }\n"
+                "  }\n");
+    else
+        dsb_put(s,
+                "  if (st0 < st1) { loadA(st0, ra0); loadB(st0, rb0); }\n"
+                "  for (u32 st = st0; st < st1; st++) {\n"
+                "    storeA(0u, st, ra0); storeB(0u, st, rb0);\n"
+                "    __syncthreads();\n"
+                "    if (st + 1u < st1) { loadA(st + 1u, ra0); loadB(st + 1u, rb0); }\n"
+                "    math(0u);\n"
+                "    /* the loads in flight are waited for by the stores, past the math */\n"
+                "    __builtin_amdgcn_sched_barrier(0);\n"
+                "    __syncthreads();\n"
+                "  }\n");
+    if (!f16) {
+        char bb[40];
+        if (pl->pack) snprintf(bb, sizeof bb, "(const char*)pk");
+        else snprintf(bb, sizeof bb, "p%u, c%u", pn->buf[1], pn->buf[1]);
+        /* the f32 instruction's pass over a tile that did not split exactly:
+         * the same groups, two k at a time, every load range-checked */
+        dsb_put(s,
+                "  bad &= 0xFFFFu;\n"
+                "  #pragma unroll\n  for (u32 b = 0; b < WM * WN; b++) {\n"
+                "    acc[b] = acc[b] + cor[b];\n"
+                "    #pragma unroll\n    for (u32 v = 0; v < 16u; v++) bad |= !(__builtin_fabsf(acc[b][v]) < __builtin_inff()) ? 1u : 0u;\n"
+                "  }\n"
+                "  u32* bf_ = (u32*)&As[0][0][0];\n"
+                "  if (tid == 0u) bf_[0] = 0u;\n"
+                "  __syncthreads();\n"
+                "  if (bad) bf_[0] = 1u;\n"
+                "  __syncthreads();\n"
+                "  if (bf_[0]) {\n"
+                "    #pragma unroll\n    for (u32 b = 0; b < WM * WN; b++) acc[b] = (f32x16){0};\n"
+                "    u32 fa[WM], fb[WN];\n"
+                "    #pragma unroll\n    for (u32 i = 0; i < WM; i++) {\n"
+                "      const u32 x = m0 + wm + i * 32u + (lane & 31u);\n"
+                "      fa[i] = row_p(x < M ? x : M - 1u); }\n"
+                "    #pragma unroll\n    for (u32 j = 0; j < WN; j++) {\n"
+                "      const u32 x = n0 + wn + j * 32u + (lane & 31u);\n"
+                "      fb[j] = row_q(x < N ? x : N - 1u); }\n"
+                "    const u32 g1 = st1 * %uu < NGRP ? st1 * %uu : NGRP;\n"
+                "    #pragma unroll 1\n"
+                "    for (u32 g = st0 * %uu; g < g1; g++) {\n"
+                "      const u32 ga = kg_p(g), gb = kg_q(g), z = kz(g);\n"
+                "      #pragma unroll 1\n"
+                "      for (u32 t = 0; t < KG; t += 2u) {\n"
+                "        const u32 kh = t + (lane >> 5);\n"
+                "        float a[WM], b[WN];\n"
+                "        #pragma unroll\n        for (u32 i = 0; i < WM; i++) a[i] = kh >= z ? ld_f32(p%u, c%u, fa[i] + ga + kh * ICP) : 0.0f;\n"
+                "        #pragma unroll\n        for (u32 j = 0; j < WN; j++) b[j] = kh >= z ? %s(%s, fb[j] + gb + kh * ICQ) : 0.0f;\n"
+                "        #pragma unroll\n        for (u32 i = 0; i < WM; i++)\n          #pragma unroll\n"
+                "          for (u32 j = 0; j < WN; j++) acc[i * WN + j] = __builtin_amdgcn_mfma_f32_32x32x2f32(%s, acc[i * WN + j], 0, 0, 0);\n"
+                "      }\n    }\n  }\n",
+                PLANE_GROUPS, PLANE_GROUPS, PLANE_GROUPS, pn->buf[0], pn->buf[0],
+                pl->pack ? "ld_f32_u" : "ld_f32", bb, pl->swap ? "b[j], a[i]" : "a[i], b[j]");
+    }
+    dsb_put(s,
+            "  #pragma unroll\n"
+            "  for (u32 blk = 0; blk < WM * WN; blk++) {\n"
+            "    const f32x16 c = acc[blk];\n"
+            "    const u32 bm = wm + (blk / WN) * 32u, bn = wn + (blk %% WN) * 32u;\n"
+            "    #pragma unroll\n"
+            "    for (u32 v = 0; v < 16u; v++) {\n"
+            "      const u32 %s = %s0 + b%s + (lane & 31u);\n"
+            "      const u32 %s = %s0 + b%s + 8u * (v >> 2) + 4u * (lane >> 5) + (v & 3u);\n"
+            "      if (m < M && n < N) {\n", pl->swap ? "m" : "n", pl->swap ? "m" : "n",
+            pl->swap ? "m" : "n", pl->swap ? "n" : "m", pl->swap ? "n" : "m", pl->swap ? "n" : "m");
+}
+
+/* What the plane-tile kernel's source needs ahead of it. */
+static void emit_plane_helpers(DSB *s, const GemmPlan *pl) {
+    const KPlane *pn = &pl->pn;
+    dsb_put(s, "typedef u32 u2_ __attribute__((ext_vector_type(2)));\ntypedef u32 u4_ __attribute__((ext_vector_type(4)));\n"
+               "typedef %s pl8_ __attribute__((ext_vector_type(8)));\n", pn->planes == 1 ? "_Float16" : "__bf16");
+    emit_kgroup_fn(s, pn, 0, pn->icoef[0], "kg_p");
+    if (pl->pack) {
+        emit_kgroup_fn(s, pn, 1, pn->icoef_q, "kg_qo");
+        dsb_put(s, "__device__ __forceinline__ u32 kg_q(u32 g) { return g * %uu; }\n", pn->G);
+    } else {
+        emit_kgroup_fn(s, pn, 1, pn->icoef[1], "kg_q");
+    }
+    /* element offset of row x of each side, ahead of its groups' */
+    dsb_put(s, "__device__ __forceinline__ u32 row_p(u32 x) { return rowb_p(gid_m(x)); }\n");
+    if (pl->pack) dsb_put(s, "__device__ __forceinline__ u32 row_q(u32 x) { return x * %uu; }\n", pn->NG * pn->G);
+    else dsb_put(s, "__device__ __forceinline__ u32 row_q(u32 x) { return rowb_q(gid_n(x)); }\n");
+    /* elements of group g that count as 0: those the group before it covers,
+     * and every one of a group past the last */
+    dsb_put(s, "__device__ __forceinline__ u32 kz(u32 g) {\n");
+    if (pn->NG % PLANE_GROUPS) dsb_put(s, "  if (g >= %uu) return %uu;\n", pn->NG, pn->G);
+    if (pn->E % pn->G) dsb_put(s, "  return g %% %uu == %uu ? %uu : 0u;\n}\n", pn->Q, pn->Q - 1, pn->Q * pn->G - pn->E);
+    else dsb_put(s, "  return 0u;\n}\n");
+    if (pn->planes != 3) return;
+    dsb_put(s,
+            "typedef __bf16 bf2_ __attribute__((ext_vector_type(2)));\ntypedef float fl2_ __attribute__((ext_vector_type(2)));\n"
+            "__device__ __forceinline__ u32 rnd2(float a, float b) {\n"
+            "  const fl2_ v = {a, b};\n"
+            "  return __builtin_bit_cast(u32, __builtin_convertvector(v, bf2_));\n}\n"
+            "__device__ __forceinline__ void split2(float a, float b, u32& h, u32& m, u32& l, u32& bad) {\n"
+            "  h = rnd2(a, b);\n"
+            "  a = a - __uint_as_float(h << 16); b = b - __uint_as_float(h & 0xFFFF0000u);\n"
+            "  m = rnd2(a, b);\n"
+            "  a = a - __uint_as_float(m << 16); b = b - __uint_as_float(m & 0xFFFF0000u);\n"
+            "  l = rnd2(a, b);\n"
+            "  bad |= __float_as_uint(a) | __float_as_uint(b);\n}\n");
+}
+
 static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const GemmPlan *pl, char *err,
                              size_t errlen) {
     /* the big tile evaluates its operands in place: separable row bases would
      * hold 16 more registers across its whole K loop (measured slower) */
     Contraction ctl = *ct_in;
-    if (pl->cfg.bm == 128 && !pl->kp.on) ctl.sep[0] = ctl.sep[1] = 0;
-    if (pl->pack) ctl.q_kmajor = 0;
+    if (!pl->cfg.direct && pl->cfg.bm == 128 && !pl->kp.on) ctl.sep[0] = ctl.sep[1] = 0;
+    if (pl->pack && pl->cfg.direct != 5) ctl.q_kmajor = 0;
     const Contraction *ct = &ctl;
     DSB s = {0};
     const TileCfg *cf = &pl->cfg;
@@ -1312,7 +1690,7 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
         emit_sep_fn(&s, side ? "rowb_q" : "rowb_p", &ct->sep_aff[side], 0);
         emit_sep_fn(&s, side ? "koff_q" : "koff_p", &ct->sep_aff[side], 1);
         if (pl->kp.on) emit_kbase_fn(&s, &pl->kp, side, side ? "kbase_q" : "kbase_p");
-        if (pl->pack && side == 1) emit_kbase_fn(&s, &pl->kpo, 1, "kbase_qo");
+        if (pl->pack && side == 1 && pl->cfg.direct != 5) emit_kbase_fn(&s, &pl->kpo, 1, "kbase_qo");
     }
     static char body[1 << 16];
     for (int side = 0; side < 2; side++) {
@@ -1328,6 +1706,29 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
         dsb_put(&s, ") {\n%s", body);
         if (op_type_is_float(k->ops[root].type)) dsb_put(&s, "  return f%u;\n}\n", root);
         else dsb_put(&s, "  return (float)n%u;\n}\n", root);
+    }
+    if (cf->direct == 5) {
+        emit_plane_helpers(&s, pl);
+        if (pl->pack) {
+            /* B's rows with their groups of k one after the other */
+            dsb_put(&s, "extern \"C\" __global__ __launch_bounds__(256) void %s_pack(", pl->name);
+            emit_params(&s, k->n_leaves);
+            dsb_put(&s, ", float* pk) {\n"
+                        "  const u32 t = blockIdx.x * 256u + threadIdx.x;\n"
+                        "  if (t >= %lluu) return;\n"
+                        "  const u32 n = t / %uu, kk = t %% %uu, g = kk / %uu, j = kk %% %uu;\n"
+                        "  pk[t] = j >= kz(g) ? ld_f32(p%u, c%u, rowb_q(gid_n(n)) + kg_qo(g) + j * %uu) : 0.0f;\n}\n",
+                    (unsigned long long)pl->pk_elems, pl->pn.NG * pl->pn.G, pl->pn.NG * pl->pn.G, pl->pn.G, pl->pn.G,
+                    ct->sep_buf[1], ct->sep_buf[1], pl->pn.icoef_q);
+        }
+        /* two waves per SIMD; one where the two LDS stages leave room for one workgroup of four */
+        dsb_put(&s, "extern \"C\" __global__ __launch_bounds__(%u) __attribute__((amdgpu_waves_per_eu(%u))) void %s(",
+                lds_threads(cf), cf->nbuf == 2 && cf->gm * cf->gn == 4 ? 1u : 2u, pl->name);
+        emit_params(&s, k->n_leaves);
+        dsb_put(&s, pl->pack ? ", float* ws, const float* pk%s) {\n" : ", float* ws%s) {\n", g_epi_params ? g_epi_params : "");
+        emit_plane_kernel(&s, ct, pl);
+        emit_store_tail(&s, k, ct, pl);
+        return s.p;
     }
     const u32 M = ct->M, N = ct->N, K = pl->kp.on ? pl->kp.Kl : ct->K;   /* the reordered (padded) K */
     const u32 tiles = pl->tiles_m * pl->tiles_n;
@@ -1579,6 +1980,7 @@ typedef struct {
  * output fused into its epilogue (fn NULL: the pair was refused). */
 #define FUSED_MAX 128
 #define EPI_SOLO_MAX_LDS 8192u
+#define PLANE_HOLD_MAX_LDS 32768u   /* plane tiles that may join a batch */
 typedef struct {
     u64 key;
     hipModule_t mod;
@@ -1610,7 +2012,8 @@ static void meta_of(const UOpKernel *k, u32 *m) {
  * can take a fused consumer: unsplit, no packed operand, f32 output, on the
  * tiled, direct or row-per-lane kernel. */
 static int plan_takes_epilogue(const GemmPlan *pl, const UOpKernel *k) {
-    return pl->splits == 1 && !pl->comb && !pl->pack && pl->cfg.direct <= 2 && k->out_dtype == DTYPE_F32;
+    return pl->splits == 1 && !pl->comb && !pl->pack && (pl->cfg.direct <= 2 || pl->cfg.direct == 5) &&
+           k->out_dtype == DTYPE_F32;
 }
 
 static DenseEntry *lookup(u64 key, const UOpKernel *k) {
@@ -1701,14 +2104,12 @@ static u64 digit_max(const Digit *d, u64 range) {
     return (range + d->div - 1) / d->div - 1;
 }
 
-static int plan_kperm(const Contraction *ct, GemmPlan *pl) {
-    KPerm *kp = &pl->kp;
-    memset(kp, 0, sizeof *kp);
-    const TileCfg *cf = &pl->cfg;
-    if (hipb.dense_nokperm || (cf->direct && cf->direct != 4)) return 0;
+/* K as its atomic digits (the finest mixed radix both separable sides' k
+ * offsets decompose into), fastest first: extents, each side's coefficients,
+ * and the largest element index a side forms. Returns their number, 0 when
+ * the offsets do not decompose. */
+static u32 k_digits(const Contraction *ct, u64 *ext, u64 (*co)[KP_MAX], u64 *maxidx) {
     const u64 K = ct->K, total = (u64)ct->M * ct->N;
-    for (int s = 0; s < 2; s++)
-        if (!ct->sep[s] || ct->sep_dt[s] != DTYPE_F32 || ct->sep_buf[s] == 0) return 0;
     /* digit boundaries of both sides' k offsets */
     u64 b[KP_MAX + 2];
     u32 nb = 0;
@@ -1729,7 +2130,6 @@ static int plan_kperm(const Contraction *ct, GemmPlan *pl) {
         if (nu == 0 || b[i] != b[nu - 1]) b[nu++] = b[i];
     if (b[nu - 1] != K) return 0;
     u32 nd = nu - 1;                      /* atomic digit j: div b[j], extent b[j+1] / b[j] */
-    u64 ext[KP_MAX], co[2][KP_MAX];
     for (u32 j = 0; j < nd; j++) {
         if (b[j + 1] % b[j]) return 0;
         ext[j] = b[j + 1] / b[j];
@@ -1752,9 +2152,23 @@ static int plan_kperm(const Contraction *ct, GemmPlan *pl) {
             if (co[s][j] > 0xFFFFFFFFull) return 0;
             mx += co[s][j] * (ext[j] - 1);
         }
-        kp->maxidx[s] = mx;
+        maxidx[s] = mx;
         if (mx > 0xFFFFFFFFull) return 0;
     }
+    return nd;
+}
+
+static int plan_kperm(const Contraction *ct, GemmPlan *pl) {
+    KPerm *kp = &pl->kp;
+    memset(kp, 0, sizeof *kp);
+    const TileCfg *cf = &pl->cfg;
+    if (hipb.dense_nokperm || (cf->direct && cf->direct != 4)) return 0;
+    const u64 K = ct->K;
+    for (int s = 0; s < 2; s++)
+        if (!ct->sep[s] || ct->sep_dt[s] != DTYPE_F32 || ct->sep_buf[s] == 0) return 0;
+    u64 ext[KP_MAX], co[2][KP_MAX];
+    const u32 nd = k_digits(ct, ext, co, kp->maxidx);
+    if (!nd) return 0;
     /* the inner digit: the longest whose extent the stage depth divides;
      * lanes along k stay coalesced only on a unit-stride inner digit, and a
      * strided one is fine only for an operand that stays in cache (weights).
@@ -1889,6 +2303,7 @@ static void plan_pack(const Contraction *ct, GemmPlan *pl) {
     }
     kp->vec[1] = !hipb.dense_novec;
     kp->maxidx[1] = (u64)kp->Kl * ct->N - 1;
+    pl->pk_elems = (u64)kp->Kl * ct->N;
 }
 
 /* K chunk per split, in stage multiples, over the K the kernel loops on (the
@@ -2053,7 +2468,205 @@ static void plan_wave_tail(GemmPlan *pl) {
     }
 }
 
+/* K groups, loads and the buffers of a plane tile, for both sides read with a
+ * single load of the same type (f32, or f16). Returns 0 when the contraction
+ * does not take one. */
+static int plan_planes(const Contraction *ct, KPlane *pn) {
+    memset(pn, 0, sizeof *pn);
+    for (int s = 0; s < 2; s++)
+        if (!ct->sep[s] || ct->sep_buf[s] == 0 || (ct->sep_dt[s] != DTYPE_F32 && ct->sep_dt[s] != DTYPE_F16)) return 0;
+    if (ct->sep_dt[0] != ct->sep_dt[1]) return 0;
+    const int f16 = ct->sep_dt[0] == DTYPE_F16;
+    const u32 es = f16 ? 2u : 4u, G = 16u / es;
+    u64 ext[KP_MAX], co[2][KP_MAX];
+    const u32 nd = k_digits(ct, ext, co, pn->maxidx);
+    if (!nd) return 0;
+    /* the loads take 32-bit byte offsets */
+    if (pn->maxidx[0] * es >= (1ull << 31) || pn->maxidx[1] * es >= (1ull << 31)) return 0;
+    /* the inner digit: the fewest elements loaded to be left out, a side with
+     * lanes along k preferring one of unit stride (a group is then one load) */
+    int best = -1;
+    double score = 0;
+    for (u32 j = 0; j < nd; j++) {
+        if (ext[j] < G) continue;
+        double c = (double)((ext[j] + G - 1) / G * G) / (double)ext[j];
+        for (int s = 0; s < 2; s++)
+            if ((s ? ct->q_kmajor : ct->p_kmajor) && co[s][j] != 1) c *= f16 ? 2.5 : 1.5;
+        if (best < 0 || c < score) {
+            best = (int)j;
+            score = c;
+        }
+    }
+    if (best < 0) return 0;
+    pn->G = G;
+    pn->E = (u32)ext[best];
+    pn->Q = (pn->E + G - 1) / G;
+    if ((u64)ct->K / pn->E * pn->Q > 0x7FFFFFFFull) return 0;
+    pn->NG = ct->K / pn->E * pn->Q;
+    pn->stages = (pn->NG + PLANE_GROUPS - 1) / PLANE_GROUPS;
+    for (u32 j = 0; j < nd; j++) {
+        if ((int)j == best) continue;
+        pn->oext[pn->ndig] = (u32)ext[j];
+        pn->ocoef[0][pn->ndig] = (u32)co[0][j];
+        pn->ocoef[1][pn->ndig] = (u32)co[1][j];
+        pn->ndig++;
+    }
+    for (int s = 0; s < 2; s++) {
+        const Aff *a = &ct->sep_aff[s];
+        const u32 nx = s ? ct->nq : ct->np, fdiv = s ? ct->qdiv[nx - 1] : ct->pdiv[nx - 1];
+        const u32 fext = s ? ct->qext[nx - 1] : ct->pext[nx - 1];
+        pn->buf[s] = ct->sep_buf[s];
+        pn->icoef[s] = (u32)co[s][best];
+        pn->kmajor[s] = s ? ct->q_kmajor : ct->p_kmajor;
+        if (!f16) {
+            pn->vec[s] = pn->kmajor[s] && pn->icoef[s] == 1;
+            continue;
+        }
+        /* 16-bit loads by two or eight start at even elements: every
+         * coefficient even but that of the dimension loaded along */
+        int ok = a->cst % 2 == 0;
+        for (u32 t = 0; t < pn->ndig; t++) ok = ok && pn->ocoef[s][t] % 2 == 0;
+        if (pn->kmajor[s]) {
+            ok = ok && pn->icoef[s] == 1 && pn->E % 2 == 0;
+            for (u32 t = 0; t < a->n; t++)
+                if (a->d[t].var == 0) ok = ok && a->coef[t] % 2 == 0;
+        } else {
+            int unit = 0;
+            ok = ok && pn->icoef[s] % 2 == 0 && fext % 2 == 0;
+            for (u32 t = 0; t < a->n; t++) {
+                if (a->d[t].var != 0) continue;
+                if (a->d[t].div == fdiv && (a->d[t].mod == 0 || a->d[t].mod == fext) && a->coef[t] == 1) unit = 1;
+                else ok = ok && a->coef[t] % 2 == 0;
+            }
+            ok = ok && unit;
+        }
+        pn->vec[s] = ok;
+    }
+    pn->planes = f16 ? 1u : 3u;
+    return 1;
+}
+
+/* Time of one stage with r workgroups of a tile on each compute unit, in ns:
+ * that of a lone workgroup (its loads, split, stores and math follow each
+ * other), or r shares of the unit's throughput. f32: measured on 1024^3 to
+ * 4096^3 (K 4096) over 64 to 4096 workgroups; the double-buffered tiles
+ * overlap a lone workgroup's steps, the others leave room for a second one. */
+static double plane_stage_ns(u32 c, u32 planes, double r, double fill) {
+    static const struct { double lone, share; } f32t[N_PLANE] = {
+        {1590, 1390}, {1920, 1420}, {1040, 910}, {1310, 770}, {740, 480}, {830, 440}};
+    static const struct { double lone, share; } f16t[N_PLANE] = {
+        {860, 750}, {1340, 650}, {700, 480}, {800, 500}, {500, 250}, {550, 250}};
+    const double l = (planes == 3 ? f32t[c].lone : f16t[c].lone) * (0.78 + 0.22 * fill), h = planes == 3 ? f32t[c].share : f16t[c].share;
+    return r * h > l ? r * h : l;
+}
+
+/* Roundings an output's sum goes through, as they add up in its error (the
+ * square of the relative error against 64-bit sums grows with their number:
+ * measured on K = 771, 1501 and 4096): the steps of one accumulator chain,
+ * and the additions that join the chains. */
+static u32 sum_roundings(u32 splits, int comb) { return splits < 2 ? 0u : comb ? splits : splits / 4u + 2u; }
+static u32 plane_roundings(const KPlane *pn, u32 st_chunk, u32 splits) {
+    return st_chunk * (pn->G * PLANE_GROUPS / 16u) * 2u / 3u + sum_roundings(splits, 0);
+}
+static u32 plan_roundings(const GemmPlan *pl, u32 K) {
+    const u32 sum = sum_roundings(pl->splits, pl->comb), kc = pl->kchunk ? pl->kchunk : K;
+    return pl->cfg.direct == 1 ? kc / (8u * pl->nw) + 2u + pl->nw + sum : kc / 2u + sum;
+}
+
+/* Time of the direct kernel, in ns: a wave's steps of 32 k, one after the
+ * other, for each wave of a SIMD. Fitted to 17 contractions of 2^20 to 2^29
+ * products (within a quarter, but for weight gradients over images, which
+ * take up to twice this); a step takes longer where K is no multiple of 4,
+ * and three times as long for f16 operands, loaded two bytes at a time. */
+static double direct_ns(const GemmPlan *pl, u32 K, u32 planes) {
+    const u32 steps = (pl->kchunk + 32u * pl->nw - 1) / (32u * pl->nw);
+    const double waves = (double)pl->tiles_m * pl->tiles_n * pl->splits * pl->nw / (4.0 * dense_cus());
+    return 2500.0 + (planes != 3 ? 7000.0 : K % 4u ? 3000.0 : 2200.0) * steps * (waves > 1.0 ? waves : 1.0) +
+           (pl->splits < 2 ? 0.0 : pl->comb ? 2000.0 : 4000.0);
+}
+
+/* The tile and K split of a plane tile with the least time, among those of no
+ * more roundings than the plan it replaces; returns that time in ns. */
+static double plan_plane_tile(const Contraction *ct, GemmPlan *pl, const KPlane *pn, u64 sig, u32 max_round) {
+    memset(pl, 0, sizeof *pl);
+    const u32 cus = dense_cus();
+    double bt = 0;
+    /* a small B side whose groups are not contiguous (the weights of a
+     * convolution, consecutive input channels a kernel's size apart) is
+     * packed: its loads touch a cache line a lane otherwise */
+    u64 pk = pn->planes == 3 && pn->kmajor[1] && pn->icoef[1] != 1 && !hipb.dense_nopack ? (u64)ct->N * pn->NG * pn->G : 0;
+    if (pk > (4u << 20)) pk = 0;
+    for (u32 c = 0; c < N_PLANE; c++) {
+        const TileCfg *cf = &CFG_PLANE[c];
+        if (hipb.dense_tile >= 12 && hipb.dense_tile != 12 + c) continue;
+        const u32 tm = (ct->M + cf->bm - 1) / cf->bm, tn = (ct->N + cf->bn - 1) / cf->bn;
+        const u64 tiles = (u64)tm * tn;
+        if (tiles > 0x7FFFFFFFull) continue;
+        for (u32 s = 1; s <= 64 && s <= pn->stages; s++) {
+            if (hipb.dense_splits ? s != hipb.dense_splits : s > 1 && pn->stages / s < 2) continue;
+            /* the partial sums fit the workspace of a dispatch without allocation */
+            if (s > 1 && (u64)s * ct->M * ct->N * 4 + pk * 4 + 512 > THVM_HIP_NOALLOC_SCRATCH_BYTES && !hipb.dense_splits) break;
+            const u32 st = (pn->stages + s - 1) / s;
+            if ((pn->stages + st - 1) / st != s) continue;
+            /* no more roundings than the plan it replaces */
+            if (!hipb.dense_splits && hipb.dense_tile < 12 && plane_roundings(pn, st, s) > max_round) continue;
+            const u64 w = tiles * s, per = (w + cus - 1) / cus;
+            double t = st * plane_stage_ns(c, pn->planes, (double)per, w < cus ? (double)w / cus : 1.0) + 3000.0;
+            if (s > 1) t += 4000.0 + (double)s * ct->M * ct->N * 8.0 / 4000.0;
+            if (!pl->cfg.bm || t < bt) {
+                bt = t;
+                pl->cfg = *cf;
+                pl->tiles_m = tm;
+                pl->tiles_n = tn;
+                pl->splits = s;
+                pl->pn = *pn;
+                pl->pn.st_chunk = st;
+            }
+        }
+    }
+    if (!pl->cfg.bm) return 0;
+    if (pk && pl->tiles_m >= PLANE_PACK_MIN_TILES) {
+        pl->pack = 1;
+        pl->pk_elems = pk;
+        pl->pn.icoef_q = pl->pn.icoef[1];
+        pl->pn.icoef[1] = 1;
+        pl->pn.vec[1] = 1;
+    }
+    pl->splits_want = pl->splits;
+    pl->nw = pl->cfg.gm * pl->cfg.gn;
+    snprintf(pl->name, sizeof pl->name, "thvm_gemm_%08x", (u32)(sig & 0xFFFFFFFFu));
+    pl->swap = !hipb.dense_noswap && ct->np > 0 && ct->pdiv[ct->np - 1] == 1 && !(ct->nq > 0 && ct->qdiv[ct->nq - 1] == 1);
+    return bt;
+}
+
+static void make_plan_f32(const Contraction *ct, GemmPlan *pl, u64 sig);
+
+/* A contraction's plan: a plane tile where both operands take one and the
+ * f32 plan is not one of the kernels shaped for it. */
 static void make_plan(const Contraction *ct, GemmPlan *pl, u64 sig) {
+    make_plan_f32(ct, pl, sig);
+    if (hipb.dense_noplanes || (hipb.dense_tile && hipb.dense_tile < 12)) return;
+    if (hipb.dense_tile < 12 &&
+        (pl->kp.on || pl->cfg.direct == 2 || pl->cfg.direct == 3 || ct->M < PLANE_MIN_SIDE || ct->N < PLANE_MIN_SIDE ||
+         (u64)ct->M * ct->N * ct->K < PLANE_MIN_WORK))
+        return;
+    KPlane pn;
+    GemmPlan pp;
+    if (!plan_planes(ct, &pn)) return;
+    const double t = plan_plane_tile(ct, &pp, &pn, sig, plan_roundings(pl, ct->K));
+    if (!pp.cfg.bm) return;
+    /* the direct kernel joins batches and sums its splits in its launch: a
+     * plane tile takes its place where the estimates are clear of each other
+     * (the 64x784x128 layer of a small network: 12.7 us, as a plane tile 5.8
+     * and a 2.9 us sum, but the step, bound by the host's launches, 38.0 us
+     * against 41.4) */
+    if (hipb.dense_tile < 12 && pl->cfg.direct == 1 &&
+        t + (pp.splits > 1 ? 3000.0 : 1000.0) >= 0.85 * direct_ns(pl, ct->K, pn.planes))
+        return;
+    *pl = pp;
+}
+
+static void make_plan_f32(const Contraction *ct, GemmPlan *pl, u64 sig) {
     static const TileCfg *forced[12] = {NULL, &CFG_BIG, &CFG_MID, &CFG_TALL, &CFG_WIDE, &CFG_DIRECT, &CFG_C64,
                                         &CFG_C64S, &CFG_SKINNY, &CFG_RED, &CFG_C64W, &CFG_WAVE};
     const int red_fits = ct->sep[0] && ct->sep[1] && ct->sep_dt[0] == DTYPE_F32 && ct->sep_dt[1] == DTYPE_F32 &&
@@ -2061,7 +2674,7 @@ static void make_plan(const Contraction *ct, GemmPlan *pl, u64 sig) {
                          (u64)ct->M * ct->N <= RED_MAX_MN && ct->N <= RED_MAX_ACC;
     /* the skinny kernel keeps N sums per lane and the outer-product one MG*N:
      * forced only where they apply */
-    const int forced_ok = hipb.dense_tile &&
+    const int forced_ok = hipb.dense_tile && hipb.dense_tile < 12 &&
                           !(hipb.dense_tile == 8 && (ct->N > SKINNY_MAX_N || (u64)ct->K * ct->N > SKINNY_MAX_KN)) &&
                           !(hipb.dense_tile == 9 && !red_fits);
     TileCfg cfg = forced_ok ? *forced[hipb.dense_tile] : pick_cfg(ct->M, ct->N, ct->K);
@@ -2177,6 +2790,13 @@ static int kperm_fits(const GemmPlan *pl, const u32 *counts, void *const *ptrs) 
     return 1;
 }
 
+/* The same for a plane tile. */
+static int planes_fit(const GemmPlan *pl, const u32 *counts, void *const *ptrs) {
+    for (int s = 0; s < 2; s++)   /* the pack kernel's loads are range-checked */
+        if (!(s && pl->pack) && (pl->pn.maxidx[s] >= counts[pl->pn.buf[s]] || ((uintptr_t)ptrs[pl->pn.buf[s]] & 3u))) return 0;
+    return 1;
+}
+
 /* Records that a program is not a contraction (the entry dense_try_dispatch
  * would leave), without dispatching it: for a program that ran only fused
  * into another launch, so that a later dispatch without allocation finds it.
@@ -2217,6 +2837,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         u32 M, N, K, sp;
         if (!dense_analyze(k, &M, &N, &K, &sp) || !recognize(k, &ct)) return 0;
         make_plan(&ct, &e->plan, uop_signature(k));
+        if (e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) make_plan_f32(&ct, &e->plan, uop_signature(k));
         if (e->plan.kp.on && !kperm_fits(&e->plan, counts, ptrs)) {
             memset(&e->plan.kp, 0, sizeof e->plan.kp);
             e->plan.pack = 0;
@@ -2275,6 +2896,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     if (!e->is_dense) return 0;
     /* buffers smaller than the plan was made for: the generated kernels */
     if (e->plan.kp.on && !kperm_fits(&e->plan, counts, ptrs)) return 0;
+    if (e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) return 0;
     for (int side = 0; side < 2; side++)
         if (e->plan.dvec[side] && ((uintptr_t)ptrs[e->plan.dvec_buf[side]] & 15u)) return 0;
     if (e->plan.cfg.direct == 2 && e->plan.ske && e->plan.skmax != ~0ull && e->plan.skmax >= counts[e->plan.skbuf])
@@ -2299,7 +2921,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     /* packed B side */
     float *pk = NULL;
     if (e->plan.pack) {
-        pk = scratch_reserve(&D.pk, (u64)e->plan.kp.maxidx[1] * sizeof(float) + sizeof(float));
+        pk = scratch_reserve(&D.pk, e->plan.pk_elems * sizeof(float));
         if (!pk) return 0;
     }
     void *params[2 * (FUSE_MAX_LEAVES + 1) + 2];
@@ -2314,7 +2936,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         void *pp[2 * (FUSE_MAX_LEAVES + 1) + 1];
         for (u32 b = 0; b < 2 * nb; b++) pp[b] = params[b];
         pp[2 * nb] = &pk;
-        const u64 kn = e->plan.kp.maxidx[1] + 1;
+        const u64 kn = e->plan.pk_elems;
         /* held: it goes out in one launch with the independent work held
          * before it (the forward convolution's pack with the padding of its
          * input), and the main kernel's launch below issues it first */
@@ -2338,7 +2960,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     /* a timed contraction (thvm_hip_time_contraction) goes out on its own,
      * between its two events */
     const int timed = hipb.time_ev[0] != NULL;
-    int held = !timed && !e->plan.pack && hipb_hold(&e->co, e->fn, tiles, e->plan.splits, params, &hm, sl != NULL,
+    int held = !timed && !e->plan.pack && !(e->plan.pn.planes && e->co.lds > PLANE_HOLD_MAX_LDS) && hipb_hold(&e->co, e->fn, tiles, e->plan.splits, params, &hm, sl != NULL,
                                                     sl ? (int)(2 * nb + 1) : -1, sl ? (u64)e->plan.splits * mn : 0);
     /* a larger launch that an elementwise consumer may still fuse into is
      * held alone if its workgroups use little LDS (the fused module adds no

@@ -66,6 +66,7 @@ typedef struct {
     int dense_nored;         /* THVM_HIP_DENSE_NORED: no outer-product reduction kernel */
     int dense_nocomb;        /* THVM_HIP_DENSE_NOCOMB: split-K partials always through a sum kernel */
     int dense_nowave;        /* THVM_HIP_DENSE_NOWAVE: no LDS-free wave-tile kernel for 64-column contractions */
+    int dense_noplanes;      /* THVM_HIP_DENSE_NOPLANES: no 16-bit plane tiles */
     int dense_notail;        /* THVM_HIP_DENSE_NOTAIL: the wave tile's last tiles are not split */
     u32 wave_tail_s;         /* THVM_HIP_WAVE_TAIL_S: waves per workgroup of the split (2, 4, 8; 0 = 4) */
     int no_fuse;             /* THVM_HIP_NO_FUSE: no elementwise consumer fused into a contraction's epilogue */
@@ -74,7 +75,8 @@ typedef struct {
     u32 dense_tile;          /* THVM_HIP_DENSE_TILE: 0 chosen, 1 128x128, 2 64x64, 3 256x32, 4 32x256, 5 direct,
                                 6 256x64, 7 128x64, 8 skinny (where N <= 16), 9 outer-product reduction
                                 (where it applies), 10 128x64 of 4 waves x 32x64, 11 wave tile (where it
-                                applies) */
+                                applies), 12.. plane tiles (where they apply: 12, 13 128x128, 14, 15
+                                128x64, 16, 17 64x64, the even ones with two LDS stages) */
     int force_interp;        /* THVM_HIP_INTERP: run generated-kernel programs on the KOp interpreter */
     int rtc_fail;            /* THVM_HIP_RTC_FAIL: treat every program compile as failed (tests) */
     u64 n_dispatch, n_compile, n_cache_hit, n_dense;
