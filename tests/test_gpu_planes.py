@@ -155,3 +155,25 @@ def test_f16_subnormals_and_infinities(hip):
     b[5] *= np.float16(512)
     a[40, 7], b[9, 20] = np.inf, np.nan
     _check(hip, "nt", prog, a, b, 130, F16)
+
+
+@pytest.mark.parametrize("what", ["plain", "inf", "tiny"])
+@pytest.mark.parametrize("case", [("nn", 2048, 1024, 2048), ("dw", 16, 128, 64, 56, 56, 3)], ids=["matmul", "weight-gradient"])
+def test_marked_tiles_take_the_f32_kernel(case, what):
+    """Contractions with a shaped f32 kernel run as a plane tile whose tiles
+    that did not split exactly that kernel computes, split over K or not."""
+    kind = case[0]
+    prog, sa, sb = ct.matmul(*case) if kind == "nn" else ct.conv(*case)
+    assert "redo_(" in _lib.dense_source(prog) and "bf_" in _lib.dense_source(prog)
+    rng = np.random.default_rng(11)
+    a, b = rng.uniform(-1, 1, sa).astype(np.float32), rng.uniform(-1, 1, sb).astype(np.float32)
+    if what == "inf":
+        a.reshape(-1)[12345] = np.inf
+    elif what == "tiny":
+        a.reshape(-1)[: a.size // 20] *= np.float32(2.0 ** -118)
+        b *= np.float32(2.0 ** 90)
+    L, saved = _init("0", "0", "0")
+    try:
+        _check(L, kind, prog, a, b, case[2] if kind == "nn" else case[1] * case[4] * case[5], F32)
+    finally:
+        _fini(L, saved)

@@ -431,6 +431,7 @@ typedef struct {
  * elements, which the group before it covers, enter as 0 on both sides. Any
  * K with a digit of at least G values splits this way. */
 #define PLANE_GROUPS 8u          /* groups per LDS stage */
+#define PLANE_SCRATCH_SPARE 65536u   /* the marks of the tiles, and alignment */
 #define PLANE_MIN_WORK (1ull << 21)
 #define PLANE_MIN_SIDE 16u       /* outputs per side: at most three quarters of a 64-wide tile empty */
 #define PLANE_PACK_MIN_TILES 8u  /* row tiles that read a packed B side */
@@ -447,13 +448,17 @@ typedef struct {
     u32 buf[2];                  /* the buffer each side loads (1 + leaf) */
     int kmajor[2];               /* lanes along k (by groups), else along the tile's rows */
     int vec[2];                  /* k-major: a group in one 16-byte load; row-major f16: two rows a load */
+    int marks;                   /* a tile that does not split exactly is marked for an f32 kernel to compute */
     u32 icoef_q;                 /* the B side's own inner coefficient where it is packed (icoef is then 1) */
 } KPlane;
 
-typedef struct {
+typedef struct GemmPlan {
     char name[48];
     TileCfg cfg;
     KPlane pn;
+    const struct GemmPlan *pt;   /* a plane tile's plan ahead of this f32 plan: its kernel (<name>_pl) runs first
+                                    and marks the tiles that did not split exactly; this plan's kernels then
+                                    compute those */
     u32 pad_a, pad_b;      /* LDS row padding (floats) of the A and B stages */
     u32 splits;
     u32 splits_want;       /* split count asked for; splits is what the K chunks give */
@@ -629,26 +634,32 @@ static void emit_sum_kernel(DSB *s_, const UOpKernel *k, const Contraction *ct, 
     out_store_fn(k, ct, fb, sizeof fb, &st);
     const u32 M = ct->M, N = ct->N;
     if (pl->splits <= 1) return;
+    /* behind a plane tile: only the outputs of the tiles computed again */
+    const char *gp = pl->pt ? ", const u32* fl_" : "";
+    char gc[128] = "";
+    if (pl->pt)
+        snprintf(gc, sizeof gc, "  if (!redo_(fl_, m / %uu * %uu, n / %uu * %uu)) return;\n", pl->cfg.bm, pl->cfg.bm, pl->cfg.bn,
+                 pl->cfg.bn);
     if (sum_per_wave(pl, (u64)M * N)) {
         /* many splits: one wavefront per output; lane l adds splits l, l+64, ...
          * in order, then a fixed shuffle tree (deterministic) */
-        dsb_put(s_, "extern \"C\" __global__ __launch_bounds__(256) void %s_sum(char* p0, u32 c0, const float* ws) {\n"
+        dsb_put(s_, "extern \"C\" __global__ __launch_bounds__(256) void %s_sum(char* p0, u32 c0, const float* ws%s) {\n"
                     "  const unsigned long long t = (unsigned long long)blockIdx.x * 4u + (threadIdx.x >> 6);\n"
                     "  const u32 lane = threadIdx.x & 63u;\n"
                     "  if (t >= %lluull) return;\n"
-                    "  const u32 %s = (u32)(t / %uu), %s = (u32)(t %% %uu);\n"
+                    "  const u32 %s = (u32)(t / %uu), %s = (u32)(t %% %uu);\n%s"
                     "  float a = 0.0f;\n"
                     "  for (u32 s = lane; s < %uu; s += 64u) a = a + ws[(unsigned long long)s * %lluull + t];\n"
                     "  a = wsum(a);\n"
                     "  if (lane == 0u) %s(p0, c0, gid_m(m) + gid_n(n), %s + a);\n}\n",
-                pl->name, (unsigned long long)M * N, pl->swap ? "n" : "m", pl->swap ? M : N, pl->swap ? "m" : "n",
-                pl->swap ? M : N, pl->splits, (unsigned long long)M * N, st, fb);
+                pl->name, gp, (unsigned long long)M * N, pl->swap ? "n" : "m", pl->swap ? M : N, pl->swap ? "m" : "n",
+                pl->swap ? M : N, gc, pl->splits, (unsigned long long)M * N, st, fb);
     } else {
         /* many outputs: a workgroup per 64 outputs, lane l of wave w adding
          * splits w, w+4, ... of output l in order; the 4 wave sums are then
          * added in a fixed order (four times the workgroups of a lane per
          * output over all splits, which is bound by its serial loads) */
-        dsb_put(s_, "extern \"C\" __global__ __launch_bounds__(256) void %s_sum(char* p0, u32 c0, const float* ws) {\n"
+        dsb_put(s_, "extern \"C\" __global__ __launch_bounds__(256) void %s_sum(char* p0, u32 c0, const float* ws%s) {\n"
                     "  __shared__ float part_[3][64];\n"
                     "  const u32 lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;\n"
                     "  const unsigned long long t = (unsigned long long)blockIdx.x * 64u + lane;\n"
@@ -661,10 +672,10 @@ static void emit_sum_kernel(DSB *s_, const UOpKernel *k, const Contraction *ct, 
                     "  __syncthreads();\n"
                     "  if (wave > 0u || t >= %lluull) return;\n"
                     "  a = ((a + part_[0][lane]) + part_[1][lane]) + part_[2][lane];\n"
-                    "  const u32 %s = (u32)(t / %uu), %s = (u32)(t %% %uu);\n"
+                    "  const u32 %s = (u32)(t / %uu), %s = (u32)(t %% %uu);\n%s"
                     "  %s(p0, c0, gid_m(m) + gid_n(n), %s + a);\n}\n",
-                pl->name, (unsigned long long)M * N, pl->splits, (unsigned long long)M * N, (unsigned long long)M * N,
-                pl->swap ? "n" : "m", pl->swap ? M : N, pl->swap ? "m" : "n", pl->swap ? M : N, st, fb);
+                pl->name, gp, (unsigned long long)M * N, pl->splits, (unsigned long long)M * N, (unsigned long long)M * N,
+                pl->swap ? "n" : "m", pl->swap ? M : N, pl->swap ? "m" : "n", pl->swap ? M : N, gc, st, fb);
     }
 }
 
@@ -1365,7 +1376,7 @@ static void emit_kgroup_fn(DSB *s, const KPlane *pn, int side, u32 icoef, const 
 
 /* One side's loader and LDS store of a plane tile. An item of a lane's work
  * is one group of one row (two rows of a paired row-major f16 side); r<x>[e]
- * holds item e's raw words, o<X>[] the byte offsets of the rows it loads. */
+ * holds item e's raw words (w<x>0, w<x>1: the lane's sets of them), o<X>[] the byte offsets of the rows it loads. */
 static void emit_plane_side(DSB *s, const Contraction *ct, const GemmPlan *pl, int side) {
     const KPlane *pn = &pl->pn;
     const TileCfg *cf = &pl->cfg;
@@ -1392,8 +1403,8 @@ static void emit_plane_side(DSB *s, const Contraction *ct, const GemmPlan *pl, i
                 X, pn->buf[side], pn->buf[side], es, pn->buf[side], es);
     char ref[40];
     snprintf(ref, sizeof ref, "u32 (&r%c)[%u][%u]", r, items, 4u * rpi);
-    dsb_put(s, "  u32 o%c[%u], r%c0[%u][%u];\n", X, nrow, r, items, 4u * rpi);
-    if (cf->nbuf == 2) dsb_put(s, "  u32 r%c1[%u][%u];\n", r, items, 4u * rpi);
+    dsb_put(s, "  u32 o%c[%u], w%c0[%u][%u];\n", X, nrow, r, items, 4u * rpi);
+    if (cf->nbuf == 2) dsb_put(s, "  u32 w%c1[%u][%u];\n", r, items, 4u * rpi);
     dsb_put(s, "  #pragma unroll\n  for (u32 e = 0; e < %uu; e++) {\n", nrow);
     if (kmaj)
         dsb_put(s, "    const u32 x = %s + tid / %uu + e * %uu;\n", side ? "n0" : "m0", PLANE_GROUPS, T / PLANE_GROUPS);
@@ -1479,7 +1490,9 @@ static void emit_plane_side(DSB *s, const Contraction *ct, const GemmPlan *pl, i
  * values below about 2^-110, whose last bits are under the bf16 range: the
  * rest they leave for the third plane does not fit its upper 16 bits (`bad`
  * collects them). A workgroup that sees either computes its tile again with
- * the f32 instruction from the operands themselves.
+ * the f32 instruction from the operands themselves; where the contraction has
+ * a shaped f32 kernel (LDS tiles with K-reordered loaders), it marks the tile
+ * instead, and that kernel, launched after it, computes the marked ones.
  *
  * One stage (PLANE_GROUPS groups of k) of LDS per workgroup; the next
  * stage's global loads are in flight across the matrix instructions. */
@@ -1487,7 +1500,7 @@ static void emit_plane_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl)
     const KPlane *pn = &pl->pn;
     const TileCfg *cf = &pl->cfg;
     const u32 WM = cf->wm_b, WN = cf->wn_b;
-    const int f16 = pn->planes == 1;
+    const int f16 = pn->planes == 1, marks = !f16 && pl->pn.marks;
     const char *op = f16 ? "__builtin_amdgcn_mfma_f32_32x32x16_f16" : "__builtin_amdgcn_mfma_f32_32x32x16_bf16";
     dsb_put(s,
             "  constexpr u32 BM = %uu, BN = %uu, BK = %uu, LD = BK + 8u, PL = %uu;\n"
@@ -1558,21 +1571,21 @@ static void emit_plane_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl)
                 "  };\n"
                 "  if (st0 < st1) {\n"
                 "    const u32 s1 = st0 + 1u < st1 ? st0 + 1u : st0;\n"
-                "    loadA(st0, ra0); loadB(st0, rb0); loadA(s1, ra1); loadB(s1, rb1);\n"
-                "    storeA(0u, st0, ra0); storeB(0u, st0, rb0);\n"
+                "    loadA(st0, wa0); loadB(st0, wb0); loadA(s1, wa1); loadB(s1, wb1);\n"
+                "    storeA(0u, st0, wa0); storeB(0u, st0, wb0);\n"
                 "    __syncthreads();\n"
                 "    for (u32 st = st0; st < st1; st += 2u) {\n"
-                "      step(st, 0u, ra1, rb1, ra0, rb0);\n"
-                "      if (st + 1u < st1) step(st + 1u, 1u, ra0, rb0, ra1, rb1);\n"
+                "      step(st, 0u, wa1, wb1, wa0, wb0);\n"
+                "      if (st + 1u < st1) step(st + 1u, 1u, wa0, wb0, wa1, wb1);\n"
                 "    }\n"
                 "  }\n");
     else
         dsb_put(s,
-                "  if (st0 < st1) { loadA(st0, ra0); loadB(st0, rb0); }\n"
+                "  if (st0 < st1) { loadA(st0, wa0); loadB(st0, wb0); }\n"
                 "  for (u32 st = st0; st < st1; st++) {\n"
-                "    storeA(0u, st, ra0); storeB(0u, st, rb0);\n"
+                "    storeA(0u, st, wa0); storeB(0u, st, wb0);\n"
                 "    __syncthreads();\n"
-                "    if (st + 1u < st1) { loadA(st + 1u, ra0); loadB(st + 1u, rb0); }\n"
+                "    if (st + 1u < st1) { loadA(st + 1u, wa0); loadB(st + 1u, wb0); }\n"
                 "    math(0u);\n"
                 "    /* the loads in flight are waited for by the stores, past the math */\n"
                 "    __builtin_amdgcn_sched_barrier(0);\n"
@@ -1594,7 +1607,11 @@ static void emit_plane_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl)
                 "  if (tid == 0u) bf_[0] = 0u;\n"
                 "  __syncthreads();\n"
                 "  if (bad) bf_[0] = 1u;\n"
-                "  __syncthreads();\n"
+                "  __syncthreads();\n");
+        if (marks)
+            dsb_put(s, "  if (tid == 0u) fl_[spl * TILES + tm * TN + tn] = bf_[0];\n");
+        else
+            dsb_put(s,
                 "  if (bf_[0]) {\n"
                 "    #pragma unroll\n    for (u32 b = 0; b < WM * WN; b++) acc[b] = (f32x16){0};\n"
                 "    u32 fa[WM], fb[WN];\n"
@@ -1670,6 +1687,48 @@ static void emit_plane_helpers(DSB *s, const GemmPlan *pl) {
             "  bad |= __float_as_uint(a) | __float_as_uint(b);\n}\n");
 }
 
+/* The plane tile's kernels: the packing of its B side, the tile, the split-K sum. */
+static void emit_plane_module(DSB *s, const UOpKernel *k, const Contraction *ct, const GemmPlan *pl) {
+    const TileCfg *cf = &pl->cfg;
+    emit_plane_helpers(s, pl);
+    if (pl->pack) {
+        /* B's rows with their groups of k one after the other */
+        dsb_put(s, "extern \"C\" __global__ __launch_bounds__(256) void %s_pack(", pl->name);
+        emit_params(s, k->n_leaves);
+        dsb_put(s, ", float* pk) {\n"
+                    "  const u32 t = blockIdx.x * 256u + threadIdx.x;\n"
+                    "  if (t >= %lluu) return;\n"
+                    "  const u32 n = t / %uu, kk = t %% %uu, g = kk / %uu, j = kk %% %uu;\n"
+                    "  pk[t] = j >= kz(g) ? ld_f32(p%u, c%u, rowb_q(gid_n(n)) + kg_qo(g) + j * %uu) : 0.0f;\n}\n",
+                (unsigned long long)pl->pk_elems, pl->pn.NG * pl->pn.G, pl->pn.NG * pl->pn.G, pl->pn.G, pl->pn.G,
+                ct->sep_buf[1], ct->sep_buf[1], pl->pn.icoef_q);
+    }
+    /* two waves per SIMD; one where the two LDS stages leave room for one workgroup of four */
+    dsb_put(s, "extern \"C\" __global__ __launch_bounds__(%u) __attribute__((amdgpu_waves_per_eu(%u))) void %s(",
+            lds_threads(cf), cf->nbuf == 2 && cf->gm * cf->gn == 4 ? 1u : 2u, pl->name);
+    emit_params(s, k->n_leaves);
+    dsb_put(s, pl->pack ? ", float* ws, const float* pk%s) {\n" : ", float* ws%s) {\n", g_epi_params ? g_epi_params : pl->pn.marks ? ", u32* fl_" : "");
+    emit_plane_kernel(s, ct, pl);
+    emit_store_tail(s, k, ct, pl);
+}
+
+/* Whether an f32 plan's kernel computes its tile at (m0, n0): the plane tile
+ * ahead of it marked one that the tile overlaps (fl_ NULL: it did not run). */
+static void emit_redo_fn(DSB *s, const Contraction *ct, const GemmPlan *pl) {
+    const GemmPlan *pt = pl->pt;
+    dsb_put(s,
+            "__device__ __forceinline__ bool redo_(const u32* fl_, u32 m0, u32 n0) {\n"
+            "  if (fl_ == nullptr) return true;\n"
+            "  const u32 m1 = (m0 + %uu < %uu ? m0 + %uu : %uu) - 1u, n1 = (n0 + %uu < %uu ? n0 + %uu : %uu) - 1u;\n"
+            "  u32 any = 0u;\n"
+            "  for (u32 s = 0; s < %uu; s++)\n"
+            "    for (u32 i = m0 / %uu; i <= m1 / %uu; i++)\n"
+            "      for (u32 j = n0 / %uu; j <= n1 / %uu; j++) any |= fl_[s * %uu + i * %uu + j];\n"
+            "  return any != 0u;\n}\n",
+            pl->cfg.bm, ct->M, pl->cfg.bm, ct->M, pl->cfg.bn, ct->N, pl->cfg.bn, ct->N, pt->splits, pt->cfg.bm,
+            pt->cfg.bm, pt->cfg.bn, pt->cfg.bn, pt->tiles_m * pt->tiles_n, pt->tiles_n);
+}
+
 static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const GemmPlan *pl, char *err,
                              size_t errlen) {
     /* the big tile evaluates its operands in place: separable row bases would
@@ -1708,28 +1767,10 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
         else dsb_put(&s, "  return (float)n%u;\n}\n", root);
     }
     if (cf->direct == 5) {
-        emit_plane_helpers(&s, pl);
-        if (pl->pack) {
-            /* B's rows with their groups of k one after the other */
-            dsb_put(&s, "extern \"C\" __global__ __launch_bounds__(256) void %s_pack(", pl->name);
-            emit_params(&s, k->n_leaves);
-            dsb_put(&s, ", float* pk) {\n"
-                        "  const u32 t = blockIdx.x * 256u + threadIdx.x;\n"
-                        "  if (t >= %lluu) return;\n"
-                        "  const u32 n = t / %uu, kk = t %% %uu, g = kk / %uu, j = kk %% %uu;\n"
-                        "  pk[t] = j >= kz(g) ? ld_f32(p%u, c%u, rowb_q(gid_n(n)) + kg_qo(g) + j * %uu) : 0.0f;\n}\n",
-                    (unsigned long long)pl->pk_elems, pl->pn.NG * pl->pn.G, pl->pn.NG * pl->pn.G, pl->pn.G, pl->pn.G,
-                    ct->sep_buf[1], ct->sep_buf[1], pl->pn.icoef_q);
-        }
-        /* two waves per SIMD; one where the two LDS stages leave room for one workgroup of four */
-        dsb_put(&s, "extern \"C\" __global__ __launch_bounds__(%u) __attribute__((amdgpu_waves_per_eu(%u))) void %s(",
-                lds_threads(cf), cf->nbuf == 2 && cf->gm * cf->gn == 4 ? 1u : 2u, pl->name);
-        emit_params(&s, k->n_leaves);
-        dsb_put(&s, pl->pack ? ", float* ws, const float* pk%s) {\n" : ", float* ws%s) {\n", g_epi_params ? g_epi_params : "");
-        emit_plane_kernel(&s, ct, pl);
-        emit_store_tail(&s, k, ct, pl);
+        emit_plane_module(&s, k, ct, pl);
         return s.p;
     }
+    if (pl->pt) emit_redo_fn(&s, ct, pl);
     const u32 M = ct->M, N = ct->N, K = pl->kp.on ? pl->kp.Kl : ct->K;   /* the reordered (padded) K */
     const u32 tiles = pl->tiles_m * pl->tiles_n;
     if (cf->direct == 2) {
@@ -1767,7 +1808,8 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
     }
     dsb_put(&s, "extern \"C\" __global__ __launch_bounds__(%u) void %s(", lds_threads(cf), pl->name);
     emit_params(&s, k->n_leaves);
-    dsb_put(&s, pl->pack ? ", float* ws, const float* pk%s) {\n" : ", float* ws%s) {\n", g_epi_params ? g_epi_params : "");
+    dsb_put(&s, pl->pack ? ", float* ws, const float* pk%s) {\n" : ", float* ws%s) {\n",
+            g_epi_params ? g_epi_params : pl->pt ? ", const u32* fl_" : "");
     dsb_put(&s,
             "  constexpr u32 BM = %u, BN = %u, BK = %u, LDA = BM + %uu, LDB = BN + %uu;\n"
             "  constexpr u32 M = %uu, N = %uu, K = %uu, TM = %uu, TN = %uu, TILES = %uu, KCH = %uu, SPLITS = %uu;\n"
@@ -1793,10 +1835,10 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
             "  { const u32 G = 8u; const u32 grp = tile / (G * TN), first = grp * G;\n"
             "    const u32 gsz = (TM - first) < G ? (TM - first) : G;\n"
             "    tm = first + (tile %% (G * TN)) %% gsz; tn = (tile %% (G * TN)) / gsz; }\n"
-            "  const u32 m0 = tm * BM, n0 = tn * BN;\n"
+            "  const u32 m0 = tm * BM, n0 = tn * BN;\n%s"
             "  const u32 kbeg = spl * KCH;\n"
             "  const u32 kend = (kbeg + KCH < K) ? kbeg + KCH : K;\n"
-            "  float ra0[%u], rb0[%u];\n", EA, EB);
+            "  float ra0[%u], rb0[%u];\n", pl->pt ? "  if (!redo_(fl_, m0, n0)) return;\n" : "", EA, EB);
     if (pl->depth == 2) dsb_put(&s, "  float ra1[%u], rb1[%u];\n", EA, EB);
     if (pl->kp.on) emit_kperm_loaders(&s, ct, pl);
     /* separable operands: per-row index bases, once per tile */
@@ -1955,6 +1997,7 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
             "      if (m < M && n < N) {\n", NB, cf->wn_b, cf->wn_b, pl->swap ? "m" : "n", pl->swap ? "m" : "n",
             pl->swap ? "m" : "n", pl->swap ? "n" : "m", pl->swap ? "n" : "m", pl->swap ? "n" : "m");
     emit_store_tail(&s, k, ct, pl);
+    if (pl->pt) emit_plane_module(&s, k, ct, pl->pt);
     return s.p;
 }
 
@@ -1969,6 +2012,8 @@ typedef struct {
     hipModule_t mod;
     hipFunction_t fn, fn_sum, fn_pack;
     GemmPlan plan;
+    GemmPlan *pt;                 /* the plane tile's plan ahead of it (plan.pt; entries move) */
+    hipFunction_t fn_pt, fn_pt_sum;
     u32 M, N;
     CoForm co, co_sum, co_pack;   /* co-launch forms of the main, split-K sum and pack kernels */
     u32 serial;                   /* unique in the process (entries move when the table grows) */
@@ -1999,6 +2044,7 @@ static struct {
     u32 cap, n;
     Scratch ws;            /* split-K partial sums */
     Scratch pk;            /* packed B operands */
+    Scratch fl;            /* a plane tile's marks for the f32 kernel behind it */
 } D;
 
 static void meta_of(const UOpKernel *k, u32 *m) {
@@ -2012,7 +2058,7 @@ static void meta_of(const UOpKernel *k, u32 *m) {
  * can take a fused consumer: unsplit, no packed operand, f32 output, on the
  * tiled, direct or row-per-lane kernel. */
 static int plan_takes_epilogue(const GemmPlan *pl, const UOpKernel *k) {
-    return pl->splits == 1 && !pl->comb && !pl->pack && (pl->cfg.direct <= 2 || pl->cfg.direct == 5) &&
+    return pl->splits == 1 && !pl->comb && !pl->pack && !pl->pt && (pl->cfg.direct <= 2 || pl->cfg.direct == 5) &&
            k->out_dtype == DTYPE_F32;
 }
 
@@ -2573,6 +2619,12 @@ static u32 plan_roundings(const GemmPlan *pl, u32 K) {
     return pl->cfg.direct == 1 ? kc / (8u * pl->nw) + 2u + pl->nw + sum : kc / 2u + sum;
 }
 
+/* Time of an f32 LDS tile, in ns: 128x128 tiles run at 125 TFLOP/s, the
+ * smaller ones at 100 (weight gradients and convolutions of 64 channels). */
+static double f32_tile_ns(const Contraction *ct, const GemmPlan *pl) {
+    return 2.0 * ct->M * ct->N * ct->K / (pl->cfg.bm == 128 && pl->cfg.bn == 128 ? 125e3 : 100e3);
+}
+
 /* Time of the direct kernel, in ns: a wave's steps of 32 k, one after the
  * other, for each wave of a SIMD. Fitted to 17 contractions of 2^20 to 2^29
  * products (within a quarter, but for weight gradients over images, which
@@ -2602,10 +2654,10 @@ static double plan_plane_tile(const Contraction *ct, GemmPlan *pl, const KPlane 
         const u32 tm = (ct->M + cf->bm - 1) / cf->bm, tn = (ct->N + cf->bn - 1) / cf->bn;
         const u64 tiles = (u64)tm * tn;
         if (tiles > 0x7FFFFFFFull) continue;
-        for (u32 s = 1; s <= 64 && s <= pn->stages; s++) {
+        for (u32 s = 1; s <= 128 && s <= pn->stages; s++) {
             if (hipb.dense_splits ? s != hipb.dense_splits : s > 1 && pn->stages / s < 2) continue;
             /* the partial sums fit the workspace of a dispatch without allocation */
-            if (s > 1 && (u64)s * ct->M * ct->N * 4 + pk * 4 + 512 > THVM_HIP_NOALLOC_SCRATCH_BYTES && !hipb.dense_splits) break;
+            if (s > 1 && (u64)s * ct->M * ct->N * 4 + pk * 4 + PLANE_SCRATCH_SPARE > THVM_HIP_NOALLOC_SCRATCH_BYTES && !hipb.dense_splits) break;
             const u32 st = (pn->stages + s - 1) / s;
             if ((pn->stages + st - 1) / st != s) continue;
             /* no more roundings than the plan it replaces */
@@ -2641,29 +2693,39 @@ static double plan_plane_tile(const Contraction *ct, GemmPlan *pl, const KPlane 
 
 static void make_plan_f32(const Contraction *ct, GemmPlan *pl, u64 sig);
 
-/* A contraction's plan: a plane tile where both operands take one and the
- * f32 plan is not one of the kernels shaped for it. */
-static void make_plan(const Contraction *ct, GemmPlan *pl, u64 sig) {
+/* A contraction's plan: a plane tile where both operands take one and it is
+ * faster than the f32 plan. In front of an f32 LDS tile it goes out as the
+ * plan's `pt` (kept in *pt), the f32 kernels following for the tiles it marks
+ * (two empty launches: 3-4 us, which the larger contractions repay: 4096^3
+ * 1040 -> 715 us, the 64-channel 3x3 weight gradient over [64,64,56,56] 144
+ * -> 112 us). The kernels shaped for narrow contractions stay. */
+static void make_plan(const Contraction *ct, GemmPlan *pl, GemmPlan *pt, u64 sig) {
     make_plan_f32(ct, pl, sig);
     if (hipb.dense_noplanes || (hipb.dense_tile && hipb.dense_tile < 12)) return;
     if (hipb.dense_tile < 12 &&
-        (pl->kp.on || pl->cfg.direct == 2 || pl->cfg.direct == 3 || ct->M < PLANE_MIN_SIDE || ct->N < PLANE_MIN_SIDE ||
+        ((pl->cfg.direct && pl->cfg.direct != 1) || ct->M < PLANE_MIN_SIDE || ct->N < PLANE_MIN_SIDE ||
          (u64)ct->M * ct->N * ct->K < PLANE_MIN_WORK))
         return;
     KPlane pn;
-    GemmPlan pp;
     if (!plan_planes(ct, &pn)) return;
-    const double t = plan_plane_tile(ct, &pp, &pn, sig, plan_roundings(pl, ct->K));
-    if (!pp.cfg.bm) return;
-    /* the direct kernel joins batches and sums its splits in its launch: a
-     * plane tile takes its place where the estimates are clear of each other
-     * (the 64x784x128 layer of a small network: 12.7 us, as a plane tile 5.8
-     * and a 2.9 us sum, but the step, bound by the host's launches, 38.0 us
-     * against 41.4) */
-    if (hipb.dense_tile < 12 && pl->cfg.direct == 1 &&
-        t + (pp.splits > 1 ? 3000.0 : 1000.0) >= 0.85 * direct_ns(pl, ct->K, pn.planes))
-        return;
-    *pl = pp;
+    const double t = plan_plane_tile(ct, pt, &pn, sig, plan_roundings(pl, ct->K));
+    if (!pt->cfg.bm) return;
+    if (hipb.dense_tile < 12) {
+        if (pl->kp.on) {
+            if (pl->pack || pt->pack || t + 6000.0 >= 0.9 * f32_tile_ns(ct, pl)) return;
+            pt->pn.marks = 1;
+            snprintf(pt->name, sizeof pt->name, "%s_pl", pl->name);
+            pl->pt = pt;
+            return;
+        }
+        /* the direct kernel joins batches and sums its splits in its launch: a
+         * plane tile takes its place where the estimates are clear of each other
+         * (the 64x784x128 layer of a small network: 12.7 us, as a plane tile 5.8
+         * and a 2.9 us sum, but the step, bound by the host's launches, 38.0 us
+         * against 41.4) */
+        if (pl->cfg.direct == 1 && t + (pt->splits > 1 ? 3000.0 : 1000.0) >= 0.85 * direct_ns(pl, ct->K, pn.planes)) return;
+    }
+    *pl = *pt;
 }
 
 static void make_plan_f32(const Contraction *ct, GemmPlan *pl, u64 sig) {
@@ -2750,8 +2812,8 @@ static void make_plan_cfg(const Contraction *ct, GemmPlan *pl, u64 sig, const Ti
 int dense_analyze(const UOpKernel *k, u32 *M, u32 *N, u32 *K, u32 *splits) {
     Contraction ct;
     if (!recognize(k, &ct)) return 0;
-    GemmPlan pl;
-    make_plan(&ct, &pl, 0);
+    GemmPlan pl, pt;
+    make_plan(&ct, &pl, &pt, 0);
     /* Matrix cores pay off once the contraction is more than a few hundred
      * thousand multiply-adds with a reduction of at least one K step: the
      * tile loaders then evaluate each operand element once instead of once
@@ -2771,8 +2833,8 @@ int dense_analyze(const UOpKernel *k, u32 *M, u32 *N, u32 *K, u32 *splits) {
 char *dense_source(const UOpKernel *k) {
     Contraction ct;
     if (!dense_analyze(k, NULL, NULL, NULL, NULL) || !recognize(k, &ct)) return NULL;
-    GemmPlan pl;
-    make_plan(&ct, &pl, uop_signature(k));
+    GemmPlan pl, pt;
+    make_plan(&ct, &pl, &pt, uop_signature(k));
     char err[128];
     return gen_gemm_source(k, &ct, &pl, err, sizeof err);
 }
@@ -2836,11 +2898,20 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         Contraction ct;
         u32 M, N, K, sp;
         if (!dense_analyze(k, &M, &N, &K, &sp) || !recognize(k, &ct)) return 0;
-        make_plan(&ct, &e->plan, uop_signature(k));
-        if (e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) make_plan_f32(&ct, &e->plan, uop_signature(k));
+        e->pt = malloc(sizeof(GemmPlan));
+        if (!e->pt) return 0;
+        make_plan(&ct, &e->plan, e->pt, uop_signature(k));
+        if ((e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) ||
+            (e->plan.pt && !planes_fit(e->plan.pt, counts, ptrs)))
+            make_plan_f32(&ct, &e->plan, uop_signature(k));
+        if (!e->plan.pt) {
+            free(e->pt);
+            e->pt = NULL;
+        }
         if (e->plan.kp.on && !kperm_fits(&e->plan, counts, ptrs)) {
             memset(&e->plan.kp, 0, sizeof e->plan.kp);
             e->plan.pack = 0;
+            e->plan.pt = NULL;
             plan_pads(&ct, &e->plan);
             plan_chunks(&ct, &e->plan);
             plan_comb(&ct, &e->plan);
@@ -2871,6 +2942,15 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
                 return 0;
             }
             co_form_make(&e->co_pack, src, nm, 256, e->fn_pack);
+        }
+        if (e->plan.pt) {
+            char nm[64];
+            snprintf(nm, sizeof nm, "%s_sum", e->pt->name);
+            if (hipModuleGetFunction(&e->fn_pt, e->mod, e->pt->name) != hipSuccess ||
+                (e->pt->splits > 1 && hipModuleGetFunction(&e->fn_pt_sum, e->mod, nm) != hipSuccess)) {
+                free(src);
+                return 0;
+            }
         }
         if (e->plan.splits > 1) {
             char nm[64];
@@ -2914,9 +2994,18 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     if (e->plan.comb && (u64)tiles * e->plan.splits <= e->cap) sl = hipb.comb_slots;
     /* split-K workspace */
     float *ws = NULL;
-    if (e->plan.splits > 1 && !sl) {
-        ws = scratch_reserve(&D.ws, (u64)e->plan.splits * e->M * e->N * sizeof(float));
+    /* a plane tile ahead of the f32 kernels: its partials (summed before
+     * theirs are written) and its marks */
+    const GemmPlan *pt = e->plan.pt && planes_fit(e->plan.pt, counts, ptrs) ? e->plan.pt : NULL;
+    const u32 wsn = pt && pt->splits > e->plan.splits ? pt->splits : e->plan.splits;
+    u32 *fl = NULL;
+    if (wsn > 1 && !sl) {
+        ws = scratch_reserve(&D.ws, (u64)wsn * e->M * e->N * sizeof(float));
         if (!ws) return 0;
+    }
+    if (pt) {
+        fl = scratch_reserve(&D.fl, (u64)pt->tiles_m * pt->tiles_n * pt->splits * sizeof(u32));
+        if (!fl) return 0;
     }
     /* packed B side */
     float *pk = NULL;
@@ -2931,7 +3020,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         params[nb + b] = &counts[b];
     }
     params[2 * nb] = &ws;
-    params[2 * nb + 1] = e->plan.comb ? (void *)&sl : (void *)&pk;
+    params[2 * nb + 1] = e->plan.pt ? (void *)&fl : e->plan.comb ? (void *)&sl : (void *)&pk;
     if (e->plan.pack) {
         void *pp[2 * (FUSE_MAX_LEAVES + 1) + 1];
         for (u32 b = 0; b < 2 * nb; b++) pp[b] = params[b];
@@ -2951,7 +3040,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     }
     /* held for a batch with the next independent dispatches (the split-K sum
      * then joins them, its main kernel going out first) */
-    const u64 mn = (u64)e->M * e->N, wsb = (u64)e->plan.splits * mn * sizeof(float);
+    const u64 mn = (u64)e->M * e->N, wsb = (u64)wsn * mn * sizeof(float);
     HbMem hm;
     hm.n = 0;
     hbm_add(&hm, ws ? (void *)ws : ptrs[0], ws ? wsb : pool_bytes(out_buf), 1);
@@ -2960,6 +3049,31 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     /* a timed contraction (thvm_hip_time_contraction) goes out on its own,
      * between its two events */
     const int timed = hipb.time_ev[0] != NULL;
+    if (e->plan.pt) {
+        if (timed) {
+            hipb_before_stream();
+            HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[0], hipb.stream));
+        }
+        int ok = 1;
+        if (pt) ok = hipb_launch_grid(e->fn_pt, pt->tiles_m * pt->tiles_n, pt->splits, lds_threads(&pt->cfg), params);
+        if (timed && pt) HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[1], hipb.stream));
+        void *p2[] = {&ptrs[0], &counts[0], &ws, &fl};
+        if (ok && pt && pt->splits > 1) {
+            const u64 per = sum_per_wave(pt, mn) ? 4 : 64;
+            ok = hipb_launch_grid(e->fn_pt_sum, (u32)((mn + per - 1) / per), 1, 256, p2);
+        }
+        if (ok) ok = hipb_launch_grid(e->fn, tiles, e->plan.splits, threads, params);
+        if (timed && !pt) HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[1], hipb.stream));
+        if (timed) {
+            hipb.time_ev[0] = hipb.time_ev[1] = NULL;
+            hipb.time_fired = 1;
+        }
+        if (ok && e->plan.splits > 1) {
+            const u64 per = sum_per_wave(&e->plan, mn) ? 4 : 64;
+            ok = hipb_launch_grid(e->fn_sum, (u32)((mn + per - 1) / per), 1, 256, p2);
+        }
+        return ok;
+    }
     int held = !timed && !e->plan.pack && !(e->plan.pn.planes && e->co.lds > PLANE_HOLD_MAX_LDS) && hipb_hold(&e->co, e->fn, tiles, e->plan.splits, params, &hm, sl != NULL,
                                                     sl ? (int)(2 * nb + 1) : -1, sl ? (u64)e->plan.splits * mn : 0);
     /* a larger launch that an elementwise consumer may still fuse into is
@@ -3012,6 +3126,7 @@ void dense_shutdown(void) {
             co_form_free(&D.tab[i].co_sum);
             co_form_free(&D.tab[i].co_pack);
             free(D.tab[i].kcopy);
+            free(D.tab[i].pt);
             free(D.tab[i].ops);
         }
         free(D.tab);
@@ -3023,6 +3138,7 @@ void dense_shutdown(void) {
     F.n = 0;
     scratch_release(&D.ws);
     scratch_release(&D.pk);
+    scratch_release(&D.fl);
     memset(&D, 0, sizeof D);
 }
 
@@ -3164,8 +3280,8 @@ char *dense_epilogue_source(const UOpKernel *k, const UOpKernel *c, u32 o_leaf, 
         snprintf(err, errlen, "not a matrix-core contraction");
         return NULL;
     }
-    GemmPlan pl;
-    make_plan(&ct, &pl, uop_signature(k));
+    GemmPlan pl, pt;
+    make_plan(&ct, &pl, &pt, uop_signature(k));
     if (!plan_takes_epilogue(&pl, k)) {
         snprintf(err, errlen, "the contraction's plan takes no epilogue");
         return NULL;
