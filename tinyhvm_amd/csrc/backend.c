@@ -1393,6 +1393,10 @@ static int hb_try_chain(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const U
     if (at < 0) return 0;
     HbEnt *h = &HB.ent[at];
     const ChainInfo *ch = h->ch;
+    /* the merged program goes after every held launch: a later step of a
+     * held sequence that reads P's output would then run before it is written */
+    for (u32 i = (u32)at + 1; i < HB.n; i++)
+        if (hbm_clash(&h->m, &HB.ent[i].m)) return 0;
     for (u32 b = 0; b < h->ch_nb; b++) {
         const HipbBuf *pb = h->ch_bufs[b] ? pool_get(h->ch_bufs[b]) : NULL;
         if (h->ch_bufs[b] && (!pb || !pb->ptr || pb->wseq > h->ch_seq)) return 0;
