@@ -1052,7 +1052,7 @@ static void read_dense_env(void) {
     if (hipb.gemm_depth > 2) hipb.gemm_depth = 0;
     e = getenv("THVM_HIP_DENSE_TILE");
     hipb.dense_tile = e ? (u32)atoi(e) : 0;
-    if (hipb.dense_tile > 17) hipb.dense_tile = 0;
+    if (hipb.dense_tile > 21) hipb.dense_tile = 0;
     hipb.dense_noplanes = env_flag("THVM_HIP_DENSE_NOPLANES");
 }
 

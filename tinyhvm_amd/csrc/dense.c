@@ -1,5 +1,5 @@
 /*
- * dense.c - routes contraction-shaped UOpKernels to f32 matrix-core kernels.
+ * dense.c - routes contraction-shaped UOpKernels to matrix-core kernels.
  *
  * The engine has no matmul or convolution op on this path: a matmul is
  * EXPAND+MUL+SUM over [M,K,N] (src/ctx/init.c:555-612) and a convolution is
@@ -26,7 +26,11 @@
  * operand values are exactly the engine's; only the summation order differs
  * (matrix-core accumulation, tolerance 1e-4 normwise).
  *
- * Kernel: 256 lanes, 128x128 output tile, K staged 16 at a time through
+ * Contractions of two plain loads of one type run on the 16-bit matrix
+ * instructions (plane tiles, and window tiles for convolutions): f16 as it
+ * is, f32 split into three bf16 planes. The others, and the small ones, on
+ * f32 kernels of several shapes; the first of them:
+ * 256 lanes, 128x128 output tile, K staged 16 at a time through
  * double-buffered LDS, each wavefront accumulating 64x64 with
  * v_mfma_f32_32x32x2_f32 (2x2 blocks). Operand tiles are loaded with the
  * lane order that is contiguous in memory for that operand (found from the
@@ -379,6 +383,14 @@ static const TileCfg CFG_PLANE[] = {
     {64, 64, 32, 1, 1, 2, 2, "plane64x64", 5, 1},
 };
 #define N_PLANE ((u32)(sizeof CFG_PLANE / sizeof CFG_PLANE[0]))
+/* Window tiles (emit_window_kernel), plane tiles of a convolution. */
+static const TileCfg CFG_WINDOW[] = {
+    {128, 128, 16, 2, 2, 2, 2, "window128x128", 5, 1},
+    {128, 64, 16, 2, 1, 2, 2, "window128x64", 5, 1},
+    {64, 64, 16, 1, 1, 2, 2, "window64x64", 5, 1},
+    {256, 64, 16, 2, 1, 4, 2, "window256x64", 5, 1},
+};
+#define N_WINDOW ((u32)(sizeof CFG_WINDOW / sizeof CFG_WINDOW[0]))
 #define RED_MAX_MN 4096
 #define RED_MIN_K 8192
 #define RED_MAX_ACC 96        /* MG * N */
@@ -418,7 +430,7 @@ typedef struct {
  * MI355X, a contraction alone): 1031x1501 over 771 86.7 -> 30.7 us, 1031x771
  * over 1501 153 -> 29 us, 2048^3 in f16 445 -> 31 us (38 -> 560 TFLOP/s); the
  * convolution of 128 channels over [32,128,28,28] 126 -> 50 us (58 -> 148
- * TFLOP/s) forward, 376 -> 47 us for its weight gradient. A full grid of
+ * TFLOP/s) forward (now a window tile), 376 -> 47 us for its weight gradient. A full grid of
  * 128x128 tiles runs at 190 TFLOP/s (six bf16 products each: 1140, where
  * hipBLASLt's largest bf16 product reaches 1209 on the same card): bound by
  * the matrix pipes' power, then by the vector instructions of the split (6
@@ -452,10 +464,32 @@ typedef struct {
     u32 icoef_q;                 /* the B side's own inner coefficient where it is packed (icoef is then 1) */
 } KPlane;
 
+/* A convolution's window tile: K is channels x taps, a tap an offset into the
+ * channel's image that is the same for every output row, so that the tile's
+ * rows read one run of positions of each channel, whatever the tap. */
+#define WINDOW_MAX_TAPS 32u
+#define WINDOW_MIN_TAPS 4u
+#define WINDOW_MIN_CHANNELS 8u
+#define WINDOW_MAX_SPAN 640u         /* positions of a tile: 60 KB of LDS */
+typedef struct {
+    u32 taps;                    /* 0: no window tile */
+    u32 off[WINDOW_MAX_TAPS];    /* a tap's offset within the image (A side) */
+    u32 qoff[WINDOW_MAX_TAPS];   /* ... and in the B side */
+    u32 E, stages;               /* channels, 16 a stage */
+    u32 cp, cq;                  /* per side: coefficient of a channel */
+    u32 U, B, sb, cst;           /* positions of an image, images, an image's stride, the first element */
+    u32 nin;                     /* the row digits within an image, fastest first */
+    u32 iext[DG_MAX], icoef[DG_MAX];
+    u32 span;                    /* LDS positions: the most a tile's rows and taps cover */
+    u32 nb;                      /* 32-column blocks of the split B side */
+    u64 pk_off;                  /* ... which starts this many floats into the pack buffer */
+} KWindow;
+
 typedef struct GemmPlan {
     char name[48];
     TileCfg cfg;
     KPlane pn;
+    KWindow wn;
     const struct GemmPlan *pt;   /* a plane tile's plan ahead of this f32 plan: its kernel (<name>_pl) runs first
                                     and marks the tiles that did not split exactly; this plan's kernels then
                                     compute those */
@@ -1133,7 +1167,7 @@ static void emit_wave_kernel(DSB *s, const UOpKernel *k, const Contraction *ct, 
     dsb_put(s, "extern \"C\" __global__ __launch_bounds__(%u) __attribute__((amdgpu_waves_per_eu(6, 8))) void %s(",
             64u * S, pl->name);
     emit_params(s, k->n_leaves);
-    dsb_put(s, ", float* ws, const float* pk%s) {\n", g_epi_params ? g_epi_params : "");
+    dsb_put(s, ", float* ws, const float* pk%s) {\n", g_epi_params ? g_epi_params : pl->pt ? ", const u32* fl_" : "");
     dsb_put(s,
             "  constexpr u32 M = %uu, N = %uu, KP = %uu, PF = %uu, TILES = %uu, ICA = %uu;\n"
             "  constexpr u32 S = %uu, FULL = %uu, NFW = FULL / S, KPC = KP / S, PFT = %uu;\n"
@@ -1158,7 +1192,7 @@ static void emit_wave_kernel(DSB *s, const UOpKernel *k, const Contraction *ct, 
             "    if (tile >= TILES) return;\n"
             "    if (TILES %% 8u == 0u) tile = (tile %% 8u) * (TILES / 8u) + tile / 8u;\n"
             "  }\n"
-            "  const u32 m0 = tile * 32u, n0 = 0u, wm = 0u, wn = 0u;\n"
+            "  const u32 m0 = tile * 32u, n0 = 0u, wm = 0u, wn = 0u;\n%s"
             "  const u32 ma = (m0 + (lane & 31u) < M) ? m0 + (lane & 31u) : M - 1u;\n"
             "  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc((void*)p%u, (short)0,\n"
             "      (int)((unsigned long long)c%u * 4ull < 0xFFFFFFFFull ? c%u * 4u : 0xFFFFFFFFu), 0x00020000);\n"
@@ -1195,7 +1229,7 @@ static void emit_wave_kernel(DSB *s, const UOpKernel *k, const Contraction *ct, 
             "    }\n"
             "  }\n",
             M, N, KPAIRS, PF, tiles, kp->icoef[0], S, pl->tail_full, pl->tail_pf ? pl->tail_pf : 1u,
-            ct->sep_buf[0], ct->sep_buf[0], ct->sep_buf[0],
+            pl->pt ? "  if (!redo_(fl_, m0, n0)) return;\n" : "", ct->sep_buf[0], ct->sep_buf[0], ct->sep_buf[0],
             kp->Kl * N, mf_a, mf_b, mf_a1, mf_b1, mf_a, mf_b, mf_a1, mf_b1);
     if (S > 1u)
         /* a tail chunk: its KPC k-pairs through the first PFT slots of the
@@ -1465,6 +1499,38 @@ static void emit_plane_side(DSB *s, const Contraction *ct, const GemmPlan *pl, i
     dsb_put(s, "    }\n  };\n");
 }
 
+/* Whether the workgroup's tile split exactly (bf_[0] is 0), once the small
+ * products are added; where an f32 kernel follows, its mark. */
+static void emit_plane_check(DSB *s, const GemmPlan *pl) {
+    dsb_put(s,
+        "  bad &= 0xFFFFu;\n"
+        "  #pragma unroll\n  for (u32 b = 0; b < WM * WN; b++) {\n"
+        "    acc[b] = acc[b] + cor[b];\n"
+        "    #pragma unroll\n    for (u32 v = 0; v < 16u; v++) bad |= !(__builtin_fabsf(acc[b][v]) < __builtin_inff()) ? 1u : 0u;\n"
+        "  }\n"
+        "  u32* bf_ = (u32*)&As[0][0][0];\n"
+        "  if (tid == 0u) bf_[0] = 0u;\n"
+        "  __syncthreads();\n"
+        "  if (bad) bf_[0] = 1u;\n"
+        "  __syncthreads();\n");
+    if (pl->pn.marks) dsb_put(s, "  if (tid == 0u) fl_[spl * TILES + tm * TN + tn] = bf_[0];\n");
+}
+
+/* The head of the stores: m, n and c[v] of each output of the wave's blocks. */
+static void emit_plane_out(DSB *s, const GemmPlan *pl) {
+    dsb_put(s,
+            "  #pragma unroll\n"
+            "  for (u32 blk = 0; blk < WM * WN; blk++) {\n"
+            "    const f32x16 c = acc[blk];\n"
+            "    const u32 bm = wm + (blk / WN) * 32u, bn = wn + (blk %% WN) * 32u;\n"
+            "    #pragma unroll\n"
+            "    for (u32 v = 0; v < 16u; v++) {\n"
+            "      const u32 %s = %s0 + b%s + (lane & 31u);\n"
+            "      const u32 %s = %s0 + b%s + 8u * (v >> 2) + 4u * (lane >> 5) + (v & 3u);\n"
+            "      if (m < M && n < N) {\n", pl->swap ? "m" : "n", pl->swap ? "m" : "n",
+            pl->swap ? "m" : "n", pl->swap ? "n" : "m", pl->swap ? "n" : "m", pl->swap ? "n" : "m");
+}
+
 /* The plane-tile kernel (CFG_PLANE): both operands go through LDS as 16-bit
  * planes, [plane][row][k], and the tile is multiplied with the 16-bit matrix
  * instructions, which run 16 times the rate of v_mfma_f32_32x32x2f32.
@@ -1595,22 +1661,10 @@ static void emit_plane_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl)
         char bb[40];
         if (pl->pack) snprintf(bb, sizeof bb, "(const char*)pk");
         else snprintf(bb, sizeof bb, "p%u, c%u", pn->buf[1], pn->buf[1]);
+        emit_plane_check(s, pl);
         /* the f32 instruction's pass over a tile that did not split exactly:
          * the same groups, two k at a time, every load range-checked */
-        dsb_put(s,
-                "  bad &= 0xFFFFu;\n"
-                "  #pragma unroll\n  for (u32 b = 0; b < WM * WN; b++) {\n"
-                "    acc[b] = acc[b] + cor[b];\n"
-                "    #pragma unroll\n    for (u32 v = 0; v < 16u; v++) bad |= !(__builtin_fabsf(acc[b][v]) < __builtin_inff()) ? 1u : 0u;\n"
-                "  }\n"
-                "  u32* bf_ = (u32*)&As[0][0][0];\n"
-                "  if (tid == 0u) bf_[0] = 0u;\n"
-                "  __syncthreads();\n"
-                "  if (bad) bf_[0] = 1u;\n"
-                "  __syncthreads();\n");
-        if (marks)
-            dsb_put(s, "  if (tid == 0u) fl_[spl * TILES + tm * TN + tn] = bf_[0];\n");
-        else
+        if (!marks)
             dsb_put(s,
                 "  if (bf_[0]) {\n"
                 "    #pragma unroll\n    for (u32 b = 0; b < WM * WN; b++) acc[b] = (f32x16){0};\n"
@@ -1637,24 +1691,192 @@ static void emit_plane_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl)
                 PLANE_GROUPS, PLANE_GROUPS, PLANE_GROUPS, pn->buf[0], pn->buf[0],
                 pl->pack ? "ld_f32_u" : "ld_f32", bb, pl->swap ? "b[j], a[i]" : "a[i], b[j]");
     }
+    emit_plane_out(s, pl);
+}
+
+/* Threads of the kernel that splits a window tile's B side: one per column
+ * and 8 channels of a stage and tap. */
+static u64 window_pack_threads(const KWindow *w) { return (u64)w->stages * w->taps * w->nb * 64u; }
+
+/* ... and its words: three planes of 16 bytes a thread, then a word a wave
+ * that is not 0 where a value did not split exactly. */
+static u64 window_pack_words(const KWindow *w) { return window_pack_threads(w) * 12u + window_pack_threads(w) / 64u; }
+
+/* The body that splits the B side, for thread t_: fragments in the order the
+ * window kernel loads them, [stage][tap][column block][plane][lane]. */
+static void emit_window_pack(DSB *s, const Contraction *ct, const KWindow *w) {
     dsb_put(s,
-            "  #pragma unroll\n"
-            "  for (u32 blk = 0; blk < WM * WN; blk++) {\n"
-            "    const f32x16 c = acc[blk];\n"
-            "    const u32 bm = wm + (blk / WN) * 32u, bn = wn + (blk %% WN) * 32u;\n"
-            "    #pragma unroll\n"
-            "    for (u32 v = 0; v < 16u; v++) {\n"
-            "      const u32 %s = %s0 + b%s + (lane & 31u);\n"
-            "      const u32 %s = %s0 + b%s + 8u * (v >> 2) + 4u * (lane >> 5) + (v & 3u);\n"
-            "      if (m < M && n < N) {\n", pl->swap ? "m" : "n", pl->swap ? "m" : "n",
-            pl->swap ? "m" : "n", pl->swap ? "n" : "m", pl->swap ? "n" : "m", pl->swap ? "n" : "m");
+            "    const u32 lane = t_ & 63u, q = t_ >> 6, n = q %% %uu * 32u + (lane & 31u);\n"
+            "    const u32 tap = q / %uu %% %uu, c0 = q / %uu * 16u + (lane >> 5) * 8u;\n"
+            "    const u32 at = rowb_q(gid_n(n < %uu ? n : %uu)) + tapq_(tap) + c0 * %uu;\n"
+            "    float x[8];\n    u32 bad = 0u;\n"
+            "    #pragma unroll\n    for (u32 j = 0; j < 8u; j++)\n"
+            "      x[j] = n < %uu && c0 + j < %uu ? ld_f32(p%u, c%u, at + j * %uu) : 0.0f;\n"
+            "    u4_ h, m, l;\n    #pragma unroll\n    for (u32 j = 0; j < 4u; j++) {\n"
+            "      u32 a, b, c; split2(x[2u * j], x[2u * j + 1u], a, b, c, bad); h[j] = a; m[j] = b; l[j] = c; }\n"
+            "    u4_* o = (u4_*)(pk + %lluu) + q * 192u + lane;\n"
+            "    o[0] = h; o[64] = m; o[128] = l;\n"
+            "    const bool any = __ballot((bad & 0xFFFFu) != 0u) != 0ull;\n"
+            "    if (lane == 0u) ((u32*)pk)[%lluu + q] = any ? 1u : 0u;\n",
+            w->nb, w->nb, w->taps, w->nb * w->taps, ct->N, ct->N - 1, w->cq, ct->N, w->E, ct->sep_buf[1], ct->sep_buf[1],
+            w->cq, (unsigned long long)w->pk_off, (unsigned long long)(w->pk_off + window_pack_threads(w) * 12u));
+}
+
+/* The window-tile kernel: the plane tile of a convolution. The rows of a tile
+ * and all taps read one run of positions of a channel's (padded) image, so a
+ * stage of 16 channels is loaded and split once and stays in LDS as
+ * [plane][8 channels][position] for all its taps: a plane tile gathers and
+ * splits every element once per tap, and those vector instructions, not the
+ * matrix ones, bound it. The images follow each other in the positions
+ * (image * U + offset), so a tile may cross from one into the next. The B
+ * side (weights) is split ahead by the pack kernel, in the fragments' order,
+ * and goes to registers directly, a tap ahead of its use; the next stage's
+ * loads are spread over the taps behind them.
+ *
+ * Measured inside a convolution's training step: 3x3, 64 channels over
+ * [64,64,56,56], the f32 wave tile 137 us, this 87 (170 TFLOP/s of f32
+ * products, 1020 of bf16 ones: near the matrix pipes' 1209 in a plain product),
+ * and 8 us for the two small launches around it; 128 channels over
+ * [32,128,28,28], the plane tile 55.6 us, this 49.6 (392 workgroups on 256
+ * compute units: a quarter of them idle at the end). */
+static void emit_window_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl) {
+    const KPlane *pn = &pl->pn;
+    const KWindow *w = &pl->wn;
+    const TileCfg *cf = &pl->cfg;
+    const u32 TT = lds_threads(cf), IT = (2u * w->span + TT - 1u) / TT;
+    char clamp[64];    /* channels past the last: a real one, against weights of 0 */
+    snprintf(clamp, sizeof clamp, "      c = c < %uu ? c : %uu;\n", w->E, w->E - 1);
+    dsb_put(s,
+            "  constexpr u32 BM = %uu, BN = %uu, M = %uu, N = %uu, TM = %uu, TN = %uu, TILES = %uu;\n"
+            "  constexpr u32 WM = %uu, WN = %uu, GN = %uu, NST = %uu, NT = %uu, SP = %uu, NB = %uu, IT = %uu, TT = %uu;\n"
+            "  __shared__ __attribute__((aligned(16))) unsigned short As[3][2][SP * 8u];\n"
+            "  const u32 tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);\n"
+            "  const u32 bid = blockIdx.x, spl = 0u;\n"
+            "  u32 tile = bid;\n"
+            "  /* consecutive tiles, whose images overlap, on one XCD */\n"
+            "  { constexpr u32 q8 = TILES / 8u, r8 = TILES %% 8u; const u32 x8 = bid %% 8u;\n"
+            "    tile = x8 * q8 + (x8 < r8 ? x8 : r8) + bid / 8u; }\n"
+            "  const u32 tm = tile / TN, tn = tile %% TN;\n"
+            "  const u32 m0 = tm * BM, n0 = tn * BN;\n"
+            "  const u32 wm = (wave / GN) * (WM * 32u), wn = (wave %% GN) * (WN * 32u);\n"
+            "  f32x16 acc[WM * WN], cor[WM * WN];\n"
+            "  #pragma unroll\n  for (u32 b = 0; b < WM * WN; b++) { acc[b] = (f32x16){0}; cor[b] = (f32x16){0}; }\n"
+            "  u32 bad = 0u;\n",
+            cf->bm, cf->bn, ct->M, ct->N, pl->tiles_m, pl->tiles_n, pl->tiles_m * pl->tiles_n, cf->wm_b, cf->wn_b, cf->gn,
+            w->stages, w->taps, w->span, w->nb, IT, TT);
+    dsb_put(s,
+            "  const __amdgpu_buffer_rsrc_t dA = __builtin_amdgcn_make_buffer_rsrc((void*)p%u, (short)0,\n"
+            "      (int)((unsigned long long)c%u * 4ull < 0xFFFFFFFFull ? c%u * 4u : 0xFFFFFFFFu), 0x00020000);\n"
+            "  const __amdgpu_buffer_rsrc_t dB = __builtin_amdgcn_make_buffer_rsrc((void*)(pk + %lluu), (short)0, (int)%lluu, 0x00020000);\n"
+            "  const u32 v0 = vpos_(m0);\n"
+            "  u32 rp[WM], oA[IT], hf[IT];\n"
+            "  #pragma unroll\n  for (u32 i = 0; i < WM; i++) {\n"
+            "    const u32 x = m0 + wm + i * 32u + (lane & 31u);\n"
+            "    rp[i] = vpos_(x < M ? x : M - 1u) - v0 + (lane >> 5) * SP; }\n"
+            "  #pragma unroll\n  for (u32 e = 0; e < IT; e++) {\n"
+            "    const u32 w0 = wave * 64u + e * TT;\n"
+            "    hf[e] = w0 / SP;    /* the wave's half of the 16 channels; 2: none */\n"
+            "    u32 v = v0 + w0 %% SP + lane;\n"
+            "    v = v < %uu ? v : %uu;\n"
+            "    oA[e] = (v / %uu * %uu + v %% %uu + %uu) * 4u; }\n"
+            "  float r[IT][8];\n"
+            "  auto loadA = [&](u32 st, u32 e) {\n"
+            "    if (hf[e] > 1u) return;\n"
+            "    #pragma unroll\n    for (u32 j = 0; j < 8u; j++) {\n"
+            "      u32 c = st * 16u + hf[e] * 8u + j;\n%s"
+            "      r[e][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(dA, (int)oA[e], (int)(c * %uu), 0)); }\n"
+            "  };\n"
+            "  auto storeA = [&](u32 e) {\n"
+            "    if (hf[e] > 1u) return;\n"
+            "    const u32 at = hf[e] * SP + (wave * 64u + e * TT) %% SP + lane;\n"
+            "    u4_ h, m, l;\n"
+            "    #pragma unroll\n    for (u32 j = 0; j < 4u; j++) {\n"
+            "      u32 a, b, c; split2(r[e][2u * j], r[e][2u * j + 1u], a, b, c, bad); h[j] = a; m[j] = b; l[j] = c; }\n"
+            "    *(u4_*)&As[0][0][at * 8u] = h; *(u4_*)&As[1][0][at * 8u] = m; *(u4_*)&As[2][0][at * 8u] = l;\n"
+            "  };\n"
+            "  auto loadB = [&](u32 q, pl8_ (&b)[3][WN]) {\n"
+            "    #pragma unroll\n    for (u32 j = 0; j < WN; j++)\n      #pragma unroll\n      for (u32 p = 0; p < 3u; p++)\n"
+            "        b[p][j] = __builtin_bit_cast(pl8_, __builtin_amdgcn_raw_buffer_load_b128(dB, (int)(lane * 16u),\n"
+            "            (int)(((q * NB + n0 / 32u + wn / 32u + j) * 3u + p) * 1024u), 0));\n"
+            "  };\n"
+            "  pl8_ b[3][WN], nb[3][WN];\n"
+            "  #pragma unroll\n  for (u32 e = 0; e < IT; e++) loadA(0u, e);\n"
+            "  loadB(0u, b);\n"
+            "  for (u32 st = 0; st < NST; st++) {\n"
+            "    #pragma unroll\n    for (u32 e = 0; e < IT; e++) storeA(e);\n"
+            "    __syncthreads();\n",
+            pn->buf[0], pn->buf[0], pn->buf[0], (unsigned long long)w->pk_off,
+            (unsigned long long)window_pack_threads(w) * 48u, w->B * w->U, w->B * w->U - 1u, w->U, w->sb, w->U, w->cst,
+            w->E % 16u ? clamp : "", w->cp * 4u);
+    static const u32 pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+    for (u32 t = 0; t < w->taps; t++) {
+        dsb_put(s, "    {\n      const u32 q = st * NT + %uu;\n      loadB(q < NST * NT ? q : NST * NT - 1u, nb);\n", t + 1);
+        for (u32 e = t * IT / w->taps; e < (t + 1) * IT / w->taps; e++) dsb_put(s, "      if (st + 1u < NST) loadA(st + 1u, %uu);\n", e);
+        dsb_put(s,
+                "      pl8_ a[3][WM];\n"
+                "      #pragma unroll\n      for (u32 p = 0; p < 3u; p++)\n        #pragma unroll\n"
+                "        for (u32 i = 0; i < WM; i++) a[p][i] = *(const pl8_*)&As[p][0][(rp[i] + %uu) * 8u];\n", w->off[t]);
+        for (u32 v = 0; v < 6; v++)
+            dsb_put(s, "      #pragma unroll\n      for (u32 i = 0; i < WM; i++)\n        #pragma unroll\n"
+                       "        for (u32 j = 0; j < WN; j++) %s[i * WN + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(%s[%u][%c], %s[%u][%c], %s[i * WN + j], 0, 0, 0);\n",
+                    v < 5u ? "cor" : "acc", pl->swap ? "b" : "a", pl->swap ? pb[v] : pa[v], pl->swap ? 'j' : 'i',
+                    pl->swap ? "a" : "b", pl->swap ? pa[v] : pb[v], pl->swap ? 'i' : 'j', v < 5u ? "cor" : "acc");
+        dsb_put(s, "      #pragma unroll\n      for (u32 p = 0; p < 3u; p++)\n        #pragma unroll\n        for (u32 j = 0; j < WN; j++) b[p][j] = nb[p][j];\n"
+                   "      __builtin_amdgcn_sched_barrier(0);\n    }\n");
+    }
+    dsb_put(s,
+            "    __syncthreads();\n  }\n"
+            "  for (u32 i = tid; i < %lluu; i += TT) bad |= ((const u32*)pk)[%lluu + i];\n",
+            (unsigned long long)window_pack_threads(w) / 64u, (unsigned long long)(w->pk_off + window_pack_threads(w) * 12u));
+    emit_plane_check(s, pl);
+    if (!pn->marks)
+        dsb_put(s,
+            "  if (bf_[0]) {\n"
+            "    #pragma unroll\n    for (u32 b = 0; b < WM * WN; b++) acc[b] = (f32x16){0};\n"
+            "    u32 fa[WM], fb[WN];\n"
+            "    #pragma unroll\n    for (u32 i = 0; i < WM; i++) {\n"
+            "      const u32 x = m0 + wm + i * 32u + (lane & 31u);\n"
+            "      fa[i] = rowb_p(gid_m(x < M ? x : M - 1u)); }\n"
+            "    #pragma unroll\n    for (u32 j = 0; j < WN; j++) {\n"
+            "      const u32 x = n0 + wn + j * 32u + (lane & 31u);\n"
+            "      fb[j] = rowb_q(gid_n(x < N ? x : N - 1u)); }\n"
+            "    #pragma unroll 1\n"
+            "    for (u32 k = 0; k < %uu; k += 2u) {\n"
+            "      const u32 kh = k + (lane >> 5), kc = kh < %uu ? kh : %uu;\n"
+            "      float x[WM], y[WN];\n"
+            "      #pragma unroll\n      for (u32 i = 0; i < WM; i++) x[i] = kh < %uu ? ld_f32(p%u, c%u, fa[i] + koff_p(kc)) : 0.0f;\n"
+            "      #pragma unroll\n      for (u32 j = 0; j < WN; j++) y[j] = kh < %uu ? ld_f32(p%u, c%u, fb[j] + koff_q(kc)) : 0.0f;\n"
+            "      #pragma unroll\n      for (u32 i = 0; i < WM; i++)\n        #pragma unroll\n"
+            "        for (u32 j = 0; j < WN; j++) acc[i * WN + j] = __builtin_amdgcn_mfma_f32_32x32x2f32(%s, acc[i * WN + j], 0, 0, 0);\n"
+            "    }\n  }\n",
+            ct->K, ct->K, ct->K - 1, ct->K, pn->buf[0], pn->buf[0], ct->K, pn->buf[1], pn->buf[1],
+            pl->swap ? "y[j], x[i]" : "x[i], y[j]");
+    emit_plane_out(s, pl);
+}
+
+/* The 16-bit vectors, and the split of two f32 values into three bf16 planes. */
+static void emit_split_helpers(DSB *s, u32 planes) {
+    dsb_put(s, "typedef u32 u2_ __attribute__((ext_vector_type(2)));\ntypedef u32 u4_ __attribute__((ext_vector_type(4)));\n"
+               "typedef %s pl8_ __attribute__((ext_vector_type(8)));\n", planes == 1 ? "_Float16" : "__bf16");
+    if (planes != 3) return;
+    dsb_put(s,
+            "typedef __bf16 bf2_ __attribute__((ext_vector_type(2)));\ntypedef float fl2_ __attribute__((ext_vector_type(2)));\n"
+            "__device__ __forceinline__ u32 rnd2(float a, float b) {\n"
+            "  const fl2_ v = {a, b};\n"
+            "  return __builtin_bit_cast(u32, __builtin_convertvector(v, bf2_));\n}\n"
+            "__device__ __forceinline__ void split2(float a, float b, u32& h, u32& m, u32& l, u32& bad) {\n"
+            "  h = rnd2(a, b);\n"
+            "  a = a - __uint_as_float(h << 16); b = b - __uint_as_float(h & 0xFFFF0000u);\n"
+            "  m = rnd2(a, b);\n"
+            "  a = a - __uint_as_float(m << 16); b = b - __uint_as_float(m & 0xFFFF0000u);\n"
+            "  l = rnd2(a, b);\n"
+            "  bad |= __float_as_uint(a) | __float_as_uint(b);\n}\n");
 }
 
 /* What the plane-tile kernel's source needs ahead of it. */
 static void emit_plane_helpers(DSB *s, const GemmPlan *pl) {
     const KPlane *pn = &pl->pn;
-    dsb_put(s, "typedef u32 u2_ __attribute__((ext_vector_type(2)));\ntypedef u32 u4_ __attribute__((ext_vector_type(4)));\n"
-               "typedef %s pl8_ __attribute__((ext_vector_type(8)));\n", pn->planes == 1 ? "_Float16" : "__bf16");
+    emit_split_helpers(s, pn->planes);
     emit_kgroup_fn(s, pn, 0, pn->icoef[0], "kg_p");
     if (pl->pack) {
         emit_kgroup_fn(s, pn, 1, pn->icoef_q, "kg_qo");
@@ -1672,19 +1894,6 @@ static void emit_plane_helpers(DSB *s, const GemmPlan *pl) {
     if (pn->NG % PLANE_GROUPS) dsb_put(s, "  if (g >= %uu) return %uu;\n", pn->NG, pn->G);
     if (pn->E % pn->G) dsb_put(s, "  return g %% %uu == %uu ? %uu : 0u;\n}\n", pn->Q, pn->Q - 1, pn->Q * pn->G - pn->E);
     else dsb_put(s, "  return 0u;\n}\n");
-    if (pn->planes != 3) return;
-    dsb_put(s,
-            "typedef __bf16 bf2_ __attribute__((ext_vector_type(2)));\ntypedef float fl2_ __attribute__((ext_vector_type(2)));\n"
-            "__device__ __forceinline__ u32 rnd2(float a, float b) {\n"
-            "  const fl2_ v = {a, b};\n"
-            "  return __builtin_bit_cast(u32, __builtin_convertvector(v, bf2_));\n}\n"
-            "__device__ __forceinline__ void split2(float a, float b, u32& h, u32& m, u32& l, u32& bad) {\n"
-            "  h = rnd2(a, b);\n"
-            "  a = a - __uint_as_float(h << 16); b = b - __uint_as_float(h & 0xFFFF0000u);\n"
-            "  m = rnd2(a, b);\n"
-            "  a = a - __uint_as_float(m << 16); b = b - __uint_as_float(m & 0xFFFF0000u);\n"
-            "  l = rnd2(a, b);\n"
-            "  bad |= __float_as_uint(a) | __float_as_uint(b);\n}\n");
 }
 
 /* The plane tile's kernels: the packing of its B side, the tile, the split-K sum. */
@@ -1712,6 +1921,41 @@ static void emit_plane_module(DSB *s, const UOpKernel *k, const Contraction *ct,
     emit_store_tail(s, k, ct, pl);
 }
 
+/* What the window tile's source needs: the split, the position of a row (its
+ * image, then its place in it) and a tap's place in the B side. */
+static void emit_window_helpers(DSB *s, const KWindow *w) {
+    emit_split_helpers(s, 3);
+    dsb_put(s, "__device__ __forceinline__ u32 vpos_(u32 x) {\n  u32 v = 0u;\n");
+    for (u32 i = 0; i < w->nin; i++) {
+        if (i + 1 < w->nin || w->B > 1) dsb_put(s, "  v += (x %% %uu) * %uu; x /= %uu;\n", w->iext[i], w->icoef[i], w->iext[i]);
+        else dsb_put(s, "  v += x * %uu;\n", w->icoef[i]);
+    }
+    dsb_put(s, w->B > 1 ? "  return v + x * %uu;\n}\n" : "  return v;\n}\n", w->U);
+    dsb_put(s, "__device__ __forceinline__ u32 tapq_(u32 t) {\n  static constexpr u32 o[%u] = {", w->taps);
+    for (u32 t = 0; t < w->taps; t++) dsb_put(s, "%s%uu", t ? ", " : "", w->qoff[t]);
+    dsb_put(s, "};\n  u32 v = 0u;\n  #pragma unroll\n  for (u32 i = 0; i < %uu; i++) v = t == i ? o[i] : v;\n  return v;\n}\n", w->taps);
+}
+
+/* The window tile's kernel, and unless the f32 plan's pack kernel does it
+ * too, the one that splits its B side. */
+static void emit_window_module(DSB *s, const UOpKernel *k, const Contraction *ct, const GemmPlan *pl) {
+    if (!pl->pn.marks) {
+        emit_window_helpers(s, &pl->wn);
+        dsb_put(s, "extern \"C\" __global__ __launch_bounds__(256) void %s_pack(", pl->name);
+        emit_params(s, k->n_leaves);
+        dsb_put(s, ", float* pk) {\n  const u32 t_ = blockIdx.x * 256u + threadIdx.x;\n  if (t_ < %lluu) {\n",
+                (unsigned long long)window_pack_threads(&pl->wn));
+        emit_window_pack(s, ct, &pl->wn);
+        dsb_put(s, "  }\n}\n");
+    }
+    dsb_put(s, "extern \"C\" __global__ __launch_bounds__(%u) __attribute__((amdgpu_waves_per_eu(%u))) void %s(",
+            lds_threads(&pl->cfg), pl->cfg.wm_b * pl->cfg.wn_b > 2 ? 2u : 3u, pl->name);
+    emit_params(s, k->n_leaves);
+    dsb_put(s, ", float* ws, const float* pk%s) {\n", pl->pn.marks ? ", u32* fl_" : "");
+    emit_window_kernel(s, ct, pl);
+    emit_store_tail(s, k, ct, pl);
+}
+
 /* Whether an f32 plan's kernel computes its tile at (m0, n0): the plane tile
  * ahead of it marked one that the tile overlaps (fl_ NULL: it did not run). */
 static void emit_redo_fn(DSB *s, const Contraction *ct, const GemmPlan *pl) {
@@ -1727,6 +1971,23 @@ static void emit_redo_fn(DSB *s, const Contraction *ct, const GemmPlan *pl) {
             "  return any != 0u;\n}\n",
             pl->cfg.bm, ct->M, pl->cfg.bm, ct->M, pl->cfg.bn, ct->N, pl->cfg.bn, ct->N, pt->splits, pt->cfg.bm,
             pt->cfg.bm, pt->cfg.bn, pt->cfg.bn, pt->tiles_m * pt->tiles_n, pt->tiles_n);
+}
+
+/* The kernels of the plane tile ahead of an f32 plan. */
+static void emit_pt_module(DSB *s, const UOpKernel *k, const Contraction *ct, const GemmPlan *pl) {
+    if (pl->pt->wn.taps) emit_window_module(s, k, ct, pl->pt);
+    else emit_plane_module(s, k, ct, pl->pt);
+}
+
+/* Threads of a plan's pack kernel, and the words of its buffer. */
+static u64 pack_threads(const GemmPlan *pl) {
+    const KWindow *w = pl->pt && pl->pt->wn.taps ? &pl->pt->wn : &pl->wn;
+    const u64 own = pl->pack && !pl->wn.taps ? pl->pk_elems : 0;
+    return w->taps ? (own + 63u) / 64u * 64u + window_pack_threads(w) : own;
+}
+static u64 pack_words(const GemmPlan *pl) {
+    const KWindow *w = pl->pt && pl->pt->wn.taps ? &pl->pt->wn : &pl->wn;
+    return w->taps ? w->pk_off + window_pack_words(w) : pl->pack ? pl->pk_elems : 0;
 }
 
 static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const GemmPlan *pl, char *err,
@@ -1767,7 +2028,8 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
         else dsb_put(&s, "  return (float)n%u;\n}\n", root);
     }
     if (cf->direct == 5) {
-        emit_plane_module(&s, k, ct, pl);
+        if (pl->wn.taps) emit_window_module(&s, k, ct, pl);
+        else emit_plane_module(&s, k, ct, pl);
         return s.p;
     }
     if (pl->pt) emit_redo_fn(&s, ct, pl);
@@ -1790,20 +2052,32 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
     const u32 BK = cf->bk;
     const u32 EA = cf->bm * BK / lds_threads(cf), EB = cf->bn * BK / lds_threads(cf);
     const u32 NB = cf->wm_b * cf->wn_b;
-    if (pl->pack) {
+    const KWindow *win = pl->pt && pl->pt->wn.taps ? &pl->pt->wn : NULL;
+    if (win) emit_window_helpers(&s, win);
+    if (pl->pack || win) {
         /* B in the reordered k order, row-major K x N (n contiguous) */
         dsb_put(&s, "extern \"C\" __global__ __launch_bounds__(256) void %s_pack(", pl->name);
         emit_params(&s, k->n_leaves);
         dsb_put(&s, ", float* pk) {\n"
-                    "  const u32 t = blockIdx.x * 256u + threadIdx.x;\n"
-                    "  if (t >= %uu) return;\n"
-                    "  const u32 k = t / %uu, n = t %% %uu;\n"
-                    "  pk[t] = (k %% %uu < %uu) ? ld_f32(p%u, c%u, kbase_qo(k) + rowb_q(gid_n(n))) : 0.0f;\n}\n",
-                pl->kp.Kl * N, N, N, pl->kp.Ep, pl->kp.E, ct->sep_buf[1], ct->sep_buf[1]);
+                    "  const u32 t = blockIdx.x * 256u + threadIdx.x;\n");
+        if (win) {   /* ... and split for the window tile, by the threads after those */
+            const u32 own = (u32)(pack_threads(pl) - window_pack_threads(win));
+            dsb_put(&s, "  if (t >= %uu) {\n    const u32 t_ = t - %uu;\n    if (t_ >= %lluu) return;\n", own, own,
+                    (unsigned long long)window_pack_threads(win));
+            emit_window_pack(&s, ct, win);
+            dsb_put(&s, "    return;\n  }\n");
+        }
+        if (pl->pack)
+            dsb_put(&s, "  if (t >= %uu) return;\n"
+                        "  const u32 k = t / %uu, n = t %% %uu;\n"
+                        "  pk[t] = (k %% %uu < %uu) ? ld_f32(p%u, c%u, kbase_qo(k) + rowb_q(gid_n(n))) : 0.0f;\n",
+                    pl->kp.Kl * N, N, N, pl->kp.Ep, pl->kp.E, ct->sep_buf[1], ct->sep_buf[1]);
+        dsb_put(&s, "}\n");
     }
     if (cf->direct == 4) {
         emit_wave_kernel(&s, k, ct, pl);
         emit_store_tail(&s, k, ct, pl);
+        if (pl->pt) emit_pt_module(&s, k, ct, pl);
         return s.p;
     }
     dsb_put(&s, "extern \"C\" __global__ __launch_bounds__(%u) void %s(", lds_threads(cf), pl->name);
@@ -1997,7 +2271,7 @@ static char *gen_gemm_source(const UOpKernel *k, const Contraction *ct_in, const
             "      if (m < M && n < N) {\n", NB, cf->wn_b, cf->wn_b, pl->swap ? "m" : "n", pl->swap ? "m" : "n",
             pl->swap ? "m" : "n", pl->swap ? "n" : "m", pl->swap ? "n" : "m", pl->swap ? "n" : "m");
     emit_store_tail(&s, k, ct, pl);
-    if (pl->pt) emit_plane_module(&s, k, ct, pl->pt);
+    if (pl->pt) emit_pt_module(&s, k, ct, pl);
     return s.p;
 }
 
@@ -2691,6 +2965,135 @@ static double plan_plane_tile(const Contraction *ct, GemmPlan *pl, const KPlane 
     return bt;
 }
 
+/* Time of a window tile, in ns: a stage's tap takes a lone workgroup `lone`,
+ * and a compute unit `share` a workgroup when it has several. Measured on 3x3
+ * convolutions of 64 channels over [64,64,56,56], 128 over [32,128,28,28] and
+ * 24 to 40 over [9,24,29,37]. */
+static double window_ns(u32 c, const KWindow *w, u64 tiles) {
+    static const struct { double lone, share; } tap[N_WINDOW] = {{680, 640}, {466, 300}, {250, 170}, {600, 600}};
+    const double per = (double)((tiles + dense_cus() - 1) / dense_cus()) * tap[c].share;
+    return w->stages * w->taps * (per > tap[c].lone ? per : tap[c].lone) + 3000.0;
+}
+
+/* A convolution's channels, taps and positions. Returns 0 where the
+ * contraction is none, or its rows do not walk one image after the other. */
+static int plan_window(const Contraction *ct, const KPlane *pn, KWindow *w) {
+    memset(w, 0, sizeof *w);
+    if (pn->planes != 3 || ct->np == 0) return 0;
+    u64 ext[KP_MAX], co[2][KP_MAX], maxidx[2];
+    const u32 nd = k_digits(ct, ext, co, maxidx);
+    int ch = -1;
+    for (u32 j = 0; j < nd; j++)
+        if (ext[j] >= WINDOW_MIN_CHANNELS && (ch < 0 || co[0][j] > co[0][ch])) ch = (int)j;
+    if (ch < 0) return 0;
+    const u64 taps = ct->K / ext[ch];
+    if (taps < WINDOW_MIN_TAPS || taps > WINDOW_MAX_TAPS) return 0;
+    u64 omax = 0;
+    for (u32 t = 0; t < taps; t++) {
+        u64 o = 0, q = 0;
+        u32 r = t;
+        for (u32 j = 0; j < nd; j++) {
+            if ((int)j == ch) continue;
+            o += r % ext[j] * co[0][j];
+            q += r % ext[j] * co[1][j];
+            r /= (u32)ext[j];
+        }
+        w->off[t] = (u32)o;
+        w->qoff[t] = (u32)q;
+        if (o > omax) omax = o;
+    }
+    w->E = (u32)ext[ch];
+    w->stages = (w->E + 15u) / 16u;
+    w->cp = (u32)co[0][ch];
+    w->cq = (u32)co[1][ch];
+    /* the coefficient of each row digit: one term of the index each */
+    const Aff *a = &ct->sep_aff[0];
+    const u64 total = (u64)ct->M * ct->N;
+    u32 rc[DG_MAX] = {0};
+    for (u32 t = 0; t < a->n; t++) {
+        if (a->d[t].var != 0) continue;
+        u32 i = 0;
+        while (i < ct->np && !(ct->pdiv[i] == a->d[t].div &&
+                               (a->d[t].mod == ct->pext[i] || (a->d[t].mod == 0 && (total - 1) / a->d[t].div < ct->pext[i])))) i++;
+        if (i == ct->np) return 0;
+        rc[i] += a->coef[t];
+    }
+    /* within an image each digit steps over all of the faster ones */
+    u64 u = 0;
+    u32 n = ct->np;
+    while (n > 0 && !(n == 1 && ct->np > 1 && rc[0] > u + omax)) {
+        n--;
+        if (rc[n] <= u) return 0;
+        w->iext[w->nin] = ct->pext[n];
+        w->icoef[w->nin++] = rc[n];
+        u += (u64)rc[n] * (ct->pext[n] - 1);
+    }
+    const u64 U = u + omax + 1;
+    w->B = n ? ct->pext[0] : 1;
+    w->sb = n ? rc[0] : 0;
+    w->cst = a->cst;
+    if (w->cst + (u64)(w->B - 1) * w->sb + U - 1 + (u64)(w->E - 1) * w->cp > pn->maxidx[0] || U * w->B >= (1ull << 31)) return 0;
+    w->U = (u32)U;
+    w->taps = (u32)taps;
+    return 1;
+}
+
+static u64 window_pos(const KWindow *w, u32 m) {
+    u64 v = 0;
+    for (u32 i = 0; i < w->nin; i++) {
+        const u32 d = i + 1 < w->nin || w->B > 1 ? m % w->iext[i] : m;
+        v += (u64)d * w->icoef[i];
+        m /= w->iext[i];
+    }
+    return w->B > 1 ? v + (u64)m * w->U : v;
+}
+
+/* The window tile of least time among those whose positions fit; returns it in ns. */
+static double plan_window_tile(const Contraction *ct, GemmPlan *pl, const KPlane *pn, const KWindow *w0, u64 sig, u64 pk_off,
+                               u32 max_round) {
+    memset(pl, 0, sizeof *pl);
+    double bt = 0;
+    u32 omax = 0;
+    for (u32 t = 0; t < w0->taps; t++) omax = w0->off[t] > omax ? w0->off[t] : omax;
+    if (hipb.dense_tile < 12 && w0->stages * w0->taps * 2u / 3u > max_round) return 0;
+    for (u32 c = 0; c < N_WINDOW; c++) {
+        const TileCfg *cf = &CFG_WINDOW[c];
+        if (hipb.dense_tile >= 12 && hipb.dense_tile != 18 + c) continue;
+        const u32 tm = (ct->M + cf->bm - 1) / cf->bm, tn = (ct->N + cf->bn - 1) / cf->bn;
+        u64 span = 0;
+        for (u32 i = 0; i < tm; i++) {
+            const u32 last = (i + 1) * cf->bm < ct->M ? (i + 1) * cf->bm - 1 : ct->M - 1;
+            const u64 n = window_pos(w0, last) - window_pos(w0, i * cf->bm) + omax + 1;
+            if (n > span) span = n;
+            if (span > WINDOW_MAX_SPAN) break;
+        }
+        span = (span + 63u) / 64u * 64u;
+        if (span > WINDOW_MAX_SPAN || (u64)tm * tn > 0x7FFFFFFFull) continue;
+        KWindow w = *w0;
+        w.span = (u32)span;
+        w.nb = tn * (cf->bn / 32u);
+        w.pk_off = pk_off;
+        if (w.pk_off + window_pack_words(&w) > (4u << 20)) continue;
+        const double t = window_ns(c, &w, (u64)tm * tn);
+        if (!pl->cfg.bm || t < bt) {
+            bt = t;
+            pl->cfg = *cf;
+            pl->tiles_m = tm;
+            pl->tiles_n = tn;
+            pl->pn = *pn;
+            pl->wn = w;
+        }
+    }
+    if (!pl->cfg.bm) return 0;
+    pl->splits = pl->splits_want = 1;
+    pl->pack = 1;
+    pl->pk_elems = pl->wn.pk_off + window_pack_words(&pl->wn);
+    pl->nw = pl->cfg.gm * pl->cfg.gn;
+    snprintf(pl->name, sizeof pl->name, "thvm_gemm_%08x", (u32)(sig & 0xFFFFFFFFu));
+    pl->swap = !hipb.dense_noswap && ct->np > 0 && ct->pdiv[ct->np - 1] == 1 && !(ct->nq > 0 && ct->qdiv[ct->nq - 1] == 1);
+    return bt;
+}
+
 static void make_plan_f32(const Contraction *ct, GemmPlan *pl, u64 sig);
 
 /* A contraction's plan: a plane tile where both operands take one and it is
@@ -2698,33 +3101,47 @@ static void make_plan_f32(const Contraction *ct, GemmPlan *pl, u64 sig);
  * plan's `pt` (kept in *pt), the f32 kernels following for the tiles it marks
  * (two empty launches: 3-4 us, which the larger contractions repay: 4096^3
  * 1040 -> 715 us, the 64-channel 3x3 weight gradient over [64,64,56,56] 144
- * -> 112 us). The kernels shaped for narrow contractions stay. */
+ * -> 112 us, its forward sum 137 -> 87 as a window tile). The kernels shaped
+ * for narrow contractions stay, but for the wave tile. */
 static void make_plan(const Contraction *ct, GemmPlan *pl, GemmPlan *pt, u64 sig) {
     make_plan_f32(ct, pl, sig);
     if (hipb.dense_noplanes || (hipb.dense_tile && hipb.dense_tile < 12)) return;
     if (hipb.dense_tile < 12 &&
-        ((pl->cfg.direct && pl->cfg.direct != 1) || ct->M < PLANE_MIN_SIDE || ct->N < PLANE_MIN_SIDE ||
+        ((pl->cfg.direct && pl->cfg.direct != 1 && pl->cfg.direct != 4) || ct->M < PLANE_MIN_SIDE || ct->N < PLANE_MIN_SIDE ||
          (u64)ct->M * ct->N * ct->K < PLANE_MIN_WORK))
         return;
     KPlane pn;
+    KWindow w;
+    GemmPlan win;
     if (!plan_planes(ct, &pn)) return;
-    const double t = plan_plane_tile(ct, pt, &pn, sig, plan_roundings(pl, ct->K));
+    const u32 rounds = plan_roundings(pl, ct->K);
+    double t = 0, tw = 0;
+    pt->cfg.bm = win.cfg.bm = 0;
+    if (hipb.dense_tile < 18 && (pl->cfg.direct != 4 || hipb.dense_tile)) t = plan_plane_tile(ct, pt, &pn, sig, rounds);
+    if ((!hipb.dense_tile || hipb.dense_tile >= 18) && plan_window(ct, &pn, &w))
+        tw = plan_window_tile(ct, &win, &pn, &w, sig, pl->kp.on && pl->pack ? (pl->pk_elems + 3u) / 4u * 4u : 0, rounds);
+    if (win.cfg.bm && (!pt->cfg.bm || tw < t)) {
+        *pt = win;
+        t = tw;
+    }
     if (!pt->cfg.bm) return;
-    if (hipb.dense_tile < 12) {
-        if (pl->kp.on) {
-            if (pl->pack || pt->pack || t + 6000.0 >= 0.9 * f32_tile_ns(ct, pl)) return;
+    if (pl->kp.on) {
+        if (hipb.dense_tile < 12 && (((pl->pack || pt->pack) && !pt->wn.taps) || t + 6000.0 >= 0.9 * f32_tile_ns(ct, pl))) return;
+        if (hipb.dense_tile < 12 || pt->wn.taps) {
             pt->pn.marks = 1;
             snprintf(pt->name, sizeof pt->name, "%s_pl", pl->name);
             pl->pt = pt;
             return;
         }
-        /* the direct kernel joins batches and sums its splits in its launch: a
-         * plane tile takes its place where the estimates are clear of each other
-         * (the 64x784x128 layer of a small network: 12.7 us, as a plane tile 5.8
-         * and a 2.9 us sum, but the step, bound by the host's launches, 38.0 us
-         * against 41.4) */
-        if (pl->cfg.direct == 1 && t + (pt->splits > 1 ? 3000.0 : 1000.0) >= 0.85 * direct_ns(pl, ct->K, pn.planes)) return;
     }
+    /* the direct kernel joins batches and sums its splits in its launch: a
+     * plane tile takes its place where the estimates are clear of each other
+     * (the 64x784x128 layer of a small network: 12.7 us, as a plane tile 5.8
+     * and a 2.9 us sum, but the step, bound by the host's launches, 38.0 us
+     * against 41.4) */
+    if (hipb.dense_tile < 12 && pl->cfg.direct == 1 &&
+        t + (pt->splits > 1 || pt->wn.taps ? 3000.0 : 1000.0) >= 0.85 * direct_ns(pl, ct->K, pn.planes))
+        return;
     *pl = *pt;
 }
 
@@ -2934,7 +3351,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         }
         co_form_make(&e->co, src, e->plan.name, dense_threads(&e->plan), e->fn);
         e->cap = rtc_capacity(e->fn, dense_threads(&e->plan));
-        if (e->plan.pack) {
+        if (pack_threads(&e->plan)) {
             char nm[64];
             snprintf(nm, sizeof nm, "%s_pack", e->plan.name);
             if (hipModuleGetFunction(&e->fn_pack, e->mod, nm) != hipSuccess) {
@@ -3009,29 +3426,30 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     }
     /* packed B side */
     float *pk = NULL;
-    if (e->plan.pack) {
-        pk = scratch_reserve(&D.pk, e->plan.pk_elems * sizeof(float));
+    if (pack_threads(&e->plan)) {
+        pk = scratch_reserve(&D.pk, pack_words(&e->plan) * sizeof(float));
         if (!pk) return 0;
     }
-    void *params[2 * (FUSE_MAX_LEAVES + 1) + 2];
+    void *params[2 * (FUSE_MAX_LEAVES + 1) + 3];
     u32 nb = k->n_leaves + 1;
     for (u32 b = 0; b < nb; b++) {
         params[b] = &ptrs[b];
         params[nb + b] = &counts[b];
     }
     params[2 * nb] = &ws;
-    params[2 * nb + 1] = e->plan.pt ? (void *)&fl : e->plan.comb ? (void *)&sl : (void *)&pk;
-    if (e->plan.pack) {
+    params[2 * nb + 1] = e->plan.pack ? (void *)&pk : e->plan.pt ? (void *)&fl : e->plan.comb ? (void *)&sl : (void *)&pk;
+    params[2 * nb + 2] = &fl;
+    if (pack_threads(&e->plan)) {
         void *pp[2 * (FUSE_MAX_LEAVES + 1) + 1];
         for (u32 b = 0; b < 2 * nb; b++) pp[b] = params[b];
         pp[2 * nb] = &pk;
-        const u64 kn = e->plan.pk_elems;
+        const u64 kn = pack_threads(&e->plan);
         /* held: it goes out in one launch with the independent work held
          * before it (the forward convolution's pack with the padding of its
          * input), and the main kernel's launch below issues it first */
         HbMem hp;
         hp.n = 0;
-        hbm_add(&hp, pk, kn * sizeof(float), 1);
+        hbm_add(&hp, pk, pack_words(&e->plan) * sizeof(float), 1);
         for (u32 i = 0; i < n_leaves && i < FUSE_MAX_LEAVES; i++)
             hbm_add(&hp, pool_ptr(leaf_bufs[i]), pool_bytes(leaf_bufs[i]), 0);
         if (!hipb_hold(&e->co_pack, e->fn_pack, (u32)((kn + 255) / 256), 1, pp, &hp, 0, -1, 0) &&
@@ -3055,14 +3473,20 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
             HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[0], hipb.stream));
         }
         int ok = 1;
-        if (pt) ok = hipb_launch_grid(e->fn_pt, pt->tiles_m * pt->tiles_n, pt->splits, lds_threads(&pt->cfg), params);
+        if (pt) {
+            void *pp[2 * (FUSE_MAX_LEAVES + 1) + 3];
+            memcpy(pp, params, sizeof pp);
+            pp[2 * nb + 1] = pt->pack ? (void *)&pk : (void *)&fl;
+            ok = hipb_launch_grid(e->fn_pt, pt->tiles_m * pt->tiles_n, pt->splits, lds_threads(&pt->cfg), pp);
+        }
         if (timed && pt) HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[1], hipb.stream));
         void *p2[] = {&ptrs[0], &counts[0], &ws, &fl};
         if (ok && pt && pt->splits > 1) {
             const u64 per = sum_per_wave(pt, mn) ? 4 : 64;
             ok = hipb_launch_grid(e->fn_pt_sum, (u32)((mn + per - 1) / per), 1, 256, p2);
         }
-        if (ok) ok = hipb_launch_grid(e->fn, tiles, e->plan.splits, threads, params);
+        const u32 gx = e->plan.tail_s ? e->plan.tail_full / e->plan.tail_s + (tiles - e->plan.tail_full) : tiles;
+        if (ok) ok = hipb_launch_grid(e->fn, gx, e->plan.splits, threads, params);
         if (timed && !pt) HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[1], hipb.stream));
         if (timed) {
             hipb.time_ev[0] = hipb.time_ev[1] = NULL;
