@@ -280,6 +280,16 @@ int  thvm_hip_batch_compile_check(const char *const *srcs, const char *const *na
  * the reference. */
 int  thvm_hip_seq_compile_check(const char *const *srcs, const char *const *names, const u32 *threads,
                                 const u32 *grid, u32 n, char *errbuf, u64 errlen);
+/* The same for the row sequence kernel of n programs over the rows of one
+ * matrix (a workgroup takes its row through them in order). A diagnostic with
+ * no counterpart in the reference. */
+int  thvm_hip_row_compile_check(const UOpKernel *const *kernels, u32 n, char *errbuf, u64 errlen);
+/* How a program takes each of its buffers (slot 0: the output) in such a
+ * sequence: 0 not at all, 1 as a matrix by its row, 2 as a vector by its row
+ * (div: gids of a row, of an elementwise program), 3 otherwise. Returns the
+ * slots written to cls and div (at most n), 0 where the program is no step
+ * of one. A diagnostic with no counterpart in the reference. */
+int  thvm_hip_row_classes(const UOpKernel *kernel, u32 *cls, u32 *div, u32 n);
 
 #ifdef __cplusplus
 }

@@ -1,0 +1,96 @@
+"""Row sequences on the GPU: every buffer as the same programs leave it when
+each is a launch of its own, bit for bit, and the softmax against float64.
+Shapes at the edges: the fewest rows, rows that are no multiple of a
+workgroup's elements, rows that threads of four straddle (not taken), long
+rows. Programs that must not be taken by row follow ones that are: a shifted
+row, a column vector of a row vector's buffer, an update in place."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests import rowprograms as rp
+from tests.rowprograms import COL, MAT, VEC
+from tinyhvm_amd import _lib, abi
+
+pytestmark = pytest.mark.gpu
+SUM, RMAX, ADD, MUL, SUB, DIV, EXP = (abi.UOP_SUM, abi.UOP_RMAX, abi.UOP_ADD, abi.UOP_MUL, abi.UOP_SUB, abi.UOP_DIV, abi.UOP_EXP)
+
+
+def two(u):
+    return lambda o, a, b: o(u, a, b)
+
+
+def one(o, v):
+    return v
+
+
+def exp_diff(o, a, b):
+    return o(EXP, o(SUB, a, b))
+
+
+def steps(m, n):
+    """(output, leaves, program): buffers by name."""
+    p = lambda *a, **kw: rp.program(m, n, *a, **kw)  # noqa: E731
+    softmax = [("mx", ["x"], p([MAT], one, reduce=RMAX)),
+               ("pick", ["h", "x"], p([MAT, MAT], two(MUL), reduce=SUM, dtypes=[rp.F16, rp.F32])),
+               ("se", ["x", "mx"], p([MAT, VEC], exp_diff, reduce=SUM)),
+               ("e", ["x", "mx"], p([MAT, VEC], exp_diff)),
+               ("s", ["e"], p([MAT], one, reduce=SUM)),
+               ("p", ["e", "s"], p([MAT, VEC], two(DIV))),
+               ("q", ["p", "c"], p([MAT, COL], two(MUL)))]
+    shifted = [("t", ["q"], p([MAT], one, reduce=SUM)),
+               ("r", ["q", "t"], p([MAT, (1, 0, 1)], two(ADD))),        # the next row's sum
+               ("u", ["q", "t"], p([(n, 1, n), VEC], two(ADD))),        # the next row
+               ("v", ["r"], p([MAT], one, reduce=RMAX)),
+               ("w", ["r", "v"], p([MAT, (0, 1, 0)], two(ADD)))]        # rows' maxima along a row
+    in_place = [("a", ["y"], p([MAT], one, reduce=SUM)),
+                ("y", ["y", "a"], p([MAT, VEC], two(ADD))),
+                ("b", ["y"], p([MAT], one, reduce=RMAX)),
+                ("x", ["y", "b"], p([MAT, VEC], two(SUB))),
+                ("a", ["x", "a"], p([MAT, VEC], two(MUL), reduce=SUM))]
+    return softmax + shifted + in_place
+
+
+def run(m, n, data):
+    L = _lib.lib()
+    L.thvm_hip_shutdown()
+    assert L.thvm_hip_init() == 0
+    ids = {}
+    for k, v in data.items():
+        ids[k] = L.thvm_hip_buf_alloc(v.nbytes)
+        L.thvm_hip_buf_write(ids[k], v.ctypes.data_as(C.c_void_p), v.nbytes)
+    st = steps(m, n)
+    for out, leaves, k in st:
+        L.thvm_hip_dispatch_uop_kernel(ids[out], (C.c_uint32 * len(leaves))(*[ids[q] for q in leaves]), len(leaves), C.byref(k), 0)
+    outs = {}
+    for k, v in data.items():
+        outs[k] = np.empty_like(v)
+        L.thvm_hip_buf_read(ids[k], outs[k].ctypes.data_as(C.c_void_p), v.nbytes)
+    assert L.thvm_hip_synchronize() == 0
+    L.thvm_hip_shutdown()
+    return outs
+
+
+@pytest.mark.parametrize("m,n", [(2, 256), (65, 260), (64, 1000), (33, 1001), (700, 1024), (4096, 1000), (2100, 5000), (300, 5000)])
+def test_rows_as_separate_launches(m, n, monkeypatch):
+    rng = np.random.default_rng(m * 7 + n)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    data = {"x": 3 * f(m, n), "h": f(m, n).astype(np.float16), "y": f(m, n), "c": f(n)}
+    data["x"][0, 5] = np.inf if m == 65 else data["x"][0, 5]
+    for k in "epqruw":
+        data[k] = np.full((m, n), -7, np.float32)
+    for k in ("mx", "pick", "se", "s", "t", "v", "a", "b"):
+        data[k] = np.full(m, -7, np.float32)
+    monkeypatch.setenv("THVM_HIP_NO_SEQ", "1")
+    want = run(m, n, data)
+    monkeypatch.delenv("THVM_HIP_NO_SEQ")
+    got = run(m, n, data)
+    for k in data:
+        assert got[k].tobytes() == want[k].tobytes(), k
+    if m != 65:
+        x = data["x"].astype(np.float64)
+        e = np.exp(x - x.max(1, keepdims=True))
+        # exp's own error, the difference's and n additions', each within 2^-24 of a term
+        err = np.abs(got["p"] - e / e.sum(1, keepdims=True)) / (e / e.sum(1, keepdims=True))
+        assert err.max() <= (n + 64) * 2.0 ** -24

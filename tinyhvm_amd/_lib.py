@@ -65,6 +65,8 @@ def lib():
         "thvm_hip_backend": (C.POINTER(abi.Backend), []),
         "thvm_hip_abi_sizes": (C.c_int, [PU32, u32]),
         "thvm_hip_kernel_source": (C.c_int, [C.POINTER(abi.UOpKernel), cp, u64, PU32, PU32]),
+        "thvm_hip_row_classes": (C.c_int, [C.POINTER(abi.UOpKernel), PU32, PU32, u32]),
+        "thvm_hip_row_compile_check": (C.c_int, [C.POINTER(C.POINTER(abi.UOpKernel)), u32, cp, u64]),
         "thvm_hip_kernel_lanes": (C.c_int, [C.POINTER(abi.UOpKernel), PU32, u32, PU32, PU32]),
         "thvm_hip_compile_check": (C.c_int, [C.POINTER(abi.UOpKernel), cp, u64]),
         "thvm_hip_dense_analyze": (C.c_int, [C.POINTER(abi.UOpKernel), PU32, PU32, PU32, PU32]),
@@ -125,7 +127,7 @@ EXPORTED = ["hip_backend"] + [
     "thvm_hip_window_analyze", "thvm_hip_window_source", "thvm_hip_window_compile_check",
     "thvm_hip_batch_compile_check", "thvm_hip_flush", "thvm_hip_epilogue_compile_check", "thvm_hip_chain_merge",
     "thvm_hip_group_compile_check", "thvm_hip_group_source", "thvm_hip_upload_source", "thvm_hip_time_contraction",
-    "thvm_hip_seq_compile_check",
+    "thvm_hip_seq_compile_check", "thvm_hip_row_classes", "thvm_hip_row_compile_check",
     "thvm_trace_load", "thvm_trace_free", "thvm_trace_count", "thvm_trace_tag",
     "thvm_trace_rec_id", "thvm_trace_rec_bytes", "thvm_trace_rec_data", "thvm_trace_rec_kernel",
     "thvm_trace_find_mark", "thvm_trace_replay", "thvm_trace_live_id", "thvm_trace_release",
@@ -148,6 +150,25 @@ def kernel_source(k: abi.UOpKernel):
     if n < 0:
         raise ValueError(text)
     return text, mode.value, vec.value
+
+
+def row_classes(k: abi.UOpKernel):
+    """How a program takes each buffer in a row sequence: (class, div) a slot,
+    class 0 unused, 1 matrix, 2 vector, 3 otherwise; [] if it is no step."""
+    cls, div = (C.c_uint32 * 65)(), (C.c_uint32 * 65)()
+    n = lib().thvm_hip_row_classes(C.byref(k), cls, div, 65)
+    return [(cls[i], div[i]) for i in range(n)]
+
+
+def row_compile_check(ks):
+    """Compile the row sequence kernel of programs without a device. Returns
+    the code-object size; raises ValueError with the reason."""
+    a = (C.POINTER(abi.UOpKernel) * len(ks))(*[C.pointer(k) for k in ks])
+    err = C.create_string_buffer(4096)
+    r = lib().thvm_hip_row_compile_check(a, len(ks), err, len(err))
+    if r < 0:
+        raise ValueError(err.value.decode())
+    return r
 
 
 def batch_compile_check(items):

@@ -105,6 +105,24 @@ static void copyq_guard_dispatch(u32 out, const u32 *leaves, u32 n) {
  * workgroup barriers or LDS of their own, none resident or held alone; if
  * one no longer qualifies when the sequence goes out (a fusion grew it), the
  * held launches go out one by one in order. */
+/* Row sequences. Reductions of a matrix's rows and elementwise programs over
+ * it (chain.c: a softmax, a cross-entropy) that depend on each other, or read
+ * the same matrix, are held too and go out as one launch with a workgroup per
+ * row, which takes its row through the programs in order, a barrier after
+ * each: what one wrote the next reads from the compute unit's or the XCD's
+ * cache. A pair of programs may share a buffer that one of them writes only
+ * if both take it by the same row (row_slots_agree). Loads of a shared row
+ * are not streamed past the caches. Every program's code is its own device
+ * function, an elementwise one called for the row's threads with the block
+ * and lane each has in its own launch: the results are those of separate
+ * launches bit for bit. Bound by the rows' bytes through the XCD's cache and
+ * the launches left: the cross-entropy head over [4096, 1000] (nine launches,
+ * 52.0 us) is four, 30.7 us (the first three reductions 10.6 us, maxima to
+ * gradient 17.3), a fused chain and its gradient over [8192, 8192], whose
+ * rows do not stay in the L2, 290 -> 276 us. A long row needs enough of them to fill the GPU:
+ * rows of more than HB_ROW_LONG elements join from HB_ROW_MANY of them. */
+#define HB_ROW_LONG 4096u
+#define HB_ROW_MANY 2048u
 #define HB_SEQ_MAX_BLOCKS 4u
 #define HB_SEQ_THREADS 256u
 #define HB_MAX 16
@@ -128,6 +146,7 @@ typedef struct {
     u32 wg;                /* a run-sum group later sums and consumers may join (1 + index into HB.wg; 0: none) */
     const void *wmax;      /* a window max a run sum over its output may take in (window.c entry; NULL: none) */
     u32 wmax_bufs[2];      /* ... its output and input */
+    const RowInfo *row;    /* a program that may be a step of a row sequence (chain.c; NULL: none) */
     u64 hid;               /* identifies the held launch while it is held */
     int seq_start;         /* reads or writes what an earlier held launch touches: starts a new step of
                               the held sequence */
@@ -141,6 +160,7 @@ static struct {
     u64 comb_used;         /* combine-area words given to the held launches */
     int flushing;
     int seq;               /* the held launches are a sequence of dependent steps (hb_seq_*) */
+    int row;               /* ... a row sequence (hb_row_*) */
     struct { u64 key; hipModule_t mod; hipFunction_t fn; u32 cap; } cache[64];
     u32 ncache;
 } HB;
@@ -262,6 +282,53 @@ static char *hb_seq_source(const HbEnt *ents, u32 n, u32 T, const char *name) {
     return src;
 }
 
+/* The row sequence kernel of n held launches over [m, cols]: workgroup r of T
+ * lanes takes row r through the programs in order (see Row sequences above). */
+static char *hb_row_source(const HbEnt *ents, u32 n, u32 cols, u32 T, const char *name) {
+    size_t cap = strlen(kgen_prelude()) + 4096;
+    for (u32 i = 0; i < n; i++) cap += strlen(ents[i].co.src) + 4 * strlen(ents[i].co.params) + 512;
+    char *src = malloc(cap);
+    if (!src) return NULL;
+    size_t w = (size_t)snprintf(src, cap, "%s\n#define ld4nt ld4\n#define ld4nt_u ld4_u\n", kgen_prelude());
+    for (u32 i = 0; i < n; i++) {
+        int seen = 0;
+        for (u32 j = 0; j < i; j++) seen |= ents[j].co.id == ents[i].co.id;
+        if (!seen) w += (size_t)snprintf(src + w, cap - w, "%s\n", ents[i].co.src);
+    }
+    w += (size_t)snprintf(src + w, cap - w, "extern \"C\" __global__ __launch_bounds__(%u) void %s(", T, name);
+    for (u32 i = 0; i < n; i++) w = hb_put_params(src, w, cap, ents[i].co.params, i, 1, i == 0);
+    w += (size_t)snprintf(src + w, cap - w, ") {\n  const u32 r_ = blockIdx.x;\n");
+    for (u32 i = 0; i < n; i++) {
+        const HbEnt *h = &ents[i];
+        if (h->row->trip) {
+            w += (size_t)snprintf(src + w, cap - w, "  co_%u::%s(r_ %% %uu, r_ / %uu, %uu, %uu, threadIdx.x", h->co.id,
+                                  h->co.name, h->gx, h->gx, h->gx, h->gy);
+        } else {
+            const u32 per = cols / h->row->per, B = h->co.threads;
+            w += (size_t)snprintf(src + w, cap - w,
+                                  "  for (u32 q_ = threadIdx.x; q_ < %uu; q_ += %uu) {\n    const u32 t_ = r_ * %uu + q_;\n"
+                                  "    co_%u::%s(t_ / %uu %% %uu, t_ / %uu / %uu, %uu, %uu, t_ %% %uu", per, T, per, h->co.id,
+                                  h->co.name, B, h->gx, B, h->gx, h->gx, h->gy, B);
+        }
+        w = hb_put_params(src, w, cap, h->co.params, i, 0, 0);
+        w += (size_t)snprintf(src + w, cap - w, h->row->trip ? ");\n" : ");\n  }\n");
+        if (i + 1 < n) w += (size_t)snprintf(src + w, cap - w, "  __syncthreads();\n");
+    }
+    snprintf(src + w, cap - w, "}\n");
+    return src;
+}
+
+static int hb_row_shape(const HbEnt *ents, u32 n, u32 *m, u32 *cols, u32 *T) {
+    for (u32 i = 0; i < n; i++)
+        if (ents[i].row && ents[i].row->trip) {
+            *m = ents[i].row->total;
+            *cols = ents[i].row->trip;
+            *T = ents[i].co.threads;
+            return 1;
+        }
+    return 0;
+}
+
 static char *hb_batch_source(const HbEnt *ents, u32 n, u32 T, const char *name) {
     size_t cap = strlen(kgen_prelude()) + 4096;
     for (u32 i = 0; i < n; i++) cap += strlen(ents[i].co.src) + 4 * strlen(ents[i].co.params) + 512;
@@ -293,7 +360,7 @@ static char *hb_batch_source(const HbEnt *ents, u32 n, u32 T, const char *name) 
 
 /* The batch kernel for the held sequence (compiled once per key) and the
  * workgroups of it the GPU holds at once (*cap). */
-static hipFunction_t hb_batch_fn(u64 key, u32 T, u32 *cap, int seq) {
+static hipFunction_t hb_batch_fn(u64 key, u32 T, u32 *cap, int seq) {   /* seq 2: a row sequence */
     *cap = 0;
     for (u32 i = 0; i < HB.ncache; i++)
         if (HB.cache[i].key == key) {
@@ -302,8 +369,11 @@ static hipFunction_t hb_batch_fn(u64 key, u32 T, u32 *cap, int seq) {
         }
     if (HB.ncache >= sizeof HB.cache / sizeof HB.cache[0]) return NULL;
     char name[48];
-    snprintf(name, sizeof name, "thvm_%s_%016llx", seq ? "seq" : "batch", (unsigned long long)key);
-    char *src = seq ? hb_seq_source(HB.ent, HB.n, T, name) : hb_batch_source(HB.ent, HB.n, T, name);
+    snprintf(name, sizeof name, "thvm_%s_%016llx", seq == 2 ? "rows" : seq ? "seq" : "batch", (unsigned long long)key);
+    u32 m, cols, rt;
+    char *src = seq == 2 ? (hb_row_shape(HB.ent, HB.n, &m, &cols, &rt) ? hb_row_source(HB.ent, HB.n, cols, T, name) : NULL)
+                : seq    ? hb_seq_source(HB.ent, HB.n, T, name)
+                         : hb_batch_source(HB.ent, HB.n, T, name);
     if (!src) return NULL;
     if (hipb.verbose) {
         fprintf(stderr, "tinyhvm-hip: %s (%u lanes):", name, T);
@@ -394,6 +464,17 @@ int thvm_hip_seq_compile_check(const char *const *srcs, const char *const *names
     return (int)r;
 }
 
+/* The held launches one by one, in order. */
+static void hb_issue_each(void) {
+    for (u32 i = 0; i < HB.n; i++) {
+        void *pv[CO_MAX_PARAMS];
+        hb_params(&HB.ent[i], pv);
+        hipb_launch(HB.ent[i].fn, HB.ent[i].gx, HB.ent[i].gy, 1, HB.ent[i].co.threads, pv);
+    }
+}
+
+static int hb_row_fits(const HbEnt *h, u32 m, u32 cols, u32 T);
+
 /* Issues the held launches: one alone as itself, several as their batch
  * kernel (or one by one if it cannot be built). */
 static void hb_flush(void) {
@@ -405,6 +486,23 @@ static void hb_flush(void) {
         void *pv[CO_MAX_PARAMS];
         hb_params(&HB.ent[0], pv);
         hipb_launch(HB.ent[0].fn, HB.ent[0].gx, HB.ent[0].gy, 1, HB.ent[0].co.threads, pv);
+    } else if (HB.row) {
+        /* a row sequence, unless a fusion has made a held launch another program */
+        u32 m = 0, cols = 0, T = 0, np = 0, cap = 0;
+        int ok = hb_row_shape(HB.ent, HB.n, &m, &cols, &T);
+        for (u32 i = 0; i < HB.n && ok; i++) ok = hb_row_fits(&HB.ent[i], m, cols, T);
+        u64 key = hb_mix(hb_mix(0x726f7773ull, T), cols);
+        for (u32 i = 0; i < HB.n; i++)
+            key = hb_mix(hb_mix(hb_mix(key, HB.ent[i].co.id), HB.ent[i].gx), HB.ent[i].gy);
+        hipFunction_t fn = ok ? hb_batch_fn(key, T, &cap, 2) : NULL;
+        if (fn) {
+            void *pv[HB_MAX * CO_MAX_PARAMS];
+            for (u32 i = 0; i < HB.n; i++) np += hb_params(&HB.ent[i], pv + np);
+            hipb_launch(fn, m, 1, 1, T, pv);
+            hipb.n_batched += HB.n;
+        } else {
+            hb_issue_each();
+        }
     } else if (HB.seq) {
         /* dependent steps: the sequence kernel, or each launch alone in order */
         const u32 T = hb_seq_threads(HB.ent, HB.n);
@@ -421,11 +519,7 @@ static void hb_flush(void) {
             hipb.n_batched += HB.n;
             hipb.n_seq += HB.n;
         } else {
-            for (u32 i = 0; i < HB.n; i++) {
-                void *pv[CO_MAX_PARAMS];
-                hb_params(&HB.ent[i], pv);
-                hipb_launch(HB.ent[i].fn, HB.ent[i].gx, HB.ent[i].gy, 1, HB.ent[i].co.threads, pv);
-            }
+            hb_issue_each();
         }
     } else {
         const u32 T = hb_threads();
@@ -454,15 +548,12 @@ static void hb_flush(void) {
             hipb_launch(fn, total, 1, 1, T, pv);
             hipb.n_batched += HB.n;
         } else {
-            for (u32 i = 0; i < HB.n; i++) {
-                void *pv[CO_MAX_PARAMS];
-                hb_params(&HB.ent[i], pv);
-                hipb_launch(HB.ent[i].fn, HB.ent[i].gx, HB.ent[i].gy, 1, HB.ent[i].co.threads, pv);
-            }
+            hb_issue_each();
         }
     }
     HB.n = 0;
     HB.seq = 0;
+    HB.row = 0;
     HB.comb_used = 0;
     memset(HB.wg_used, 0, sizeof HB.wg_used);
     HB.flushing = 0;
@@ -524,10 +615,69 @@ static int hb_seq_join(const HbEnt *h) {
     return lds <= HB_MAX_LDS;
 }
 
+/* whether a held launch is a step of a row sequence over [m, cols] by T lanes */
+static int hb_row_fits(const HbEnt *h, u32 m, u32 cols, u32 T) {
+    const RowInfo *ri = h->row;
+    if (!ri || hipb.no_seq || h->solo || h->resident || h->fz_key || h->wg || h->wmax || !h->co.src) return 0;
+    if (ri->trip)   /* a workgroup a row */
+        return ri->total == m && ri->trip == cols && (u64)h->gx * h->gy == m && h->co.threads == T;
+    /* threads that each take their own gids, the row's all its own */
+    return (u64)m * cols == ri->total && ri->per && cols % ri->per == 0 && h->co.lane_free;
+}
+
+/* the address range of a held program's buffer slot (its parameters begin
+ * with the pointers, then the element counts) */
+static void hb_row_slot(const HbEnt *h, u32 s, u64 *lo, u64 *hi) {
+    u32 c;
+    memcpy(lo, h->args + 8u * s, 8);
+    memcpy(&c, h->args + 8u * (h->row->n_leaves + 1u) + 4u * s, 4);
+    *hi = *lo + (u64)c * (h->row->f16[s] ? 2u : 4u);
+}
+
+/* whether b may follow a in a row sequence of cols columns; *gain is set
+ * where it reads what a wrote, or both take one matrix */
+static int hb_row_pair(const HbEnt *a, const HbEnt *b, u32 cols, int *gain) {
+    for (u32 i = 0; i <= a->row->n_leaves; i++) {
+        if (a->row->cls[i] == ROW_UNUSED) continue;
+        u64 alo, ahi;
+        hb_row_slot(a, i, &alo, &ahi);
+        for (u32 j = 0; j <= b->row->n_leaves; j++) {
+            if (b->row->cls[j] == ROW_UNUSED) continue;
+            u64 blo, bhi;
+            hb_row_slot(b, j, &blo, &bhi);
+            if (!hb_overlap(alo, ahi, blo, bhi)) continue;
+            const int wr = ((a->row->writes >> i) & 1u) || ((b->row->writes >> j) & 1u);
+            const int agree = alo == blo && row_slots_agree(a->row, i, b->row, j, cols);
+            if (wr && !agree) return 0;
+            if (agree && (wr || a->row->cls[i] == ROW_MATRIX)) *gain = 1;
+        }
+    }
+    return 1;
+}
+
+/* whether h may follow the held launches in a row sequence, and gains by it */
+static int hb_row_join(const HbEnt *h) {
+    u32 m, cols, T;
+    if (HB.n == 0 || HB.n >= HB_MAX) return 0;
+    if (!hb_row_shape(HB.ent, HB.n, &m, &cols, &T) && !hb_row_shape(h, 1, &m, &cols, &T)) return 0;
+    if (!hb_row_fits(h, m, cols, T) || (cols > HB_ROW_LONG && m < HB_ROW_MANY)) return 0;
+    u32 lds = h->co.lds;
+    int gain = 0;
+    for (u32 i = 0; i < HB.n; i++) {
+        if (!hb_row_fits(&HB.ent[i], m, cols, T) || !hb_row_pair(&HB.ent[i], h, cols, &gain)) return 0;
+        lds += HB.ent[i].co.lds;
+    }
+    return gain && lds <= HB_MAX_LDS;
+}
+
+/* a reduction of too many workgroups for a batch, held for a row sequence */
+static int hb_row_only(const HbEnt *h) { return h->row && h->row->trip && (u64)h->gx * h->gy > HB_MAX_BLOCKS; }
+
 /* why h cannot join the held launches as they are (NULL: it can) */
 static const char *hb_joins(const HbEnt *h) {
     if (HB.n >= HB_MAX) return "batch full";
     if (h->solo || (HB.n && HB.ent[0].solo)) return "held alone";
+    if (HB.n && hb_row_only(h)) return "rows";
     u32 T = h->co.threads, lds = h->co.lds, blocks = h->gx * h->gy;
     int resident = h->resident;
     /* the batch kernel holds no more waves at once than its most demanding
@@ -536,6 +686,7 @@ static const char *hb_joins(const HbEnt *h) {
     for (u32 i = 0; i < HB.n; i++) {
         const HbEnt *o = &HB.ent[i];
         if (hbm_clash(&h->m, &o->m)) return "memory";
+        if (hb_row_only(o)) return "rows";
         if (o->co.threads > T) T = o->co.threads;
         lds += o->co.lds;
         blocks += o->gx * o->gy;
@@ -550,33 +701,26 @@ static const char *hb_joins(const HbEnt *h) {
 }
 
 static int hb_hold(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *const *params, const HbMem *m,
-                   int resident, int comb_param, u64 comb_words, int solo);
+                   int resident, int comb_param, u64 comb_words, int solo, const RowInfo *row);
 
 int hipb_hold(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *const *params, const HbMem *m,
               int resident, int comb_param, u64 comb_words) {
-    return hb_hold(cf, fn, gx, gy, params, m, resident, comb_param, comb_words, 0);
+    return hb_hold(cf, fn, gx, gy, params, m, resident, comb_param, comb_words, 0, NULL);
 }
 
 int hipb_hold_solo(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *const *params, const HbMem *m) {
     if (hipb.no_fuse) return 0;
-    return hb_hold(cf, fn, gx, gy, params, m, 0, -1, 0, 1);
-}
-
-/* A chainable generated program (chain.c) of any grid size: held (and batched like
- * the small ones) so that a consumer of its output can fuse after it. */
-static int hb_hold_large(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *const *params, const HbMem *m) {
-    if (hipb.no_fuse) return 0;
-    return hb_hold(cf, fn, gx, gy, params, m, 0, -1, 0, 2);
+    return hb_hold(cf, fn, gx, gy, params, m, 0, -1, 0, 1, NULL);
 }
 
 int hipb_hold_large(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *const *params, const HbMem *m,
                     int resident, int comb_param, u64 comb_words) {
     if (hipb.no_fuse) return 0;
-    return hb_hold(cf, fn, gx, gy, params, m, resident, comb_param, comb_words, 2);
+    return hb_hold(cf, fn, gx, gy, params, m, resident, comb_param, comb_words, 2, NULL);
 }
 
 static int hb_hold(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *const *params, const HbMem *m,
-                   int resident, int comb_param, u64 comb_words, int solo) {
+                   int resident, int comb_param, u64 comb_words, int solo, const RowInfo *row) {
     if (!cf || !cf->src || hipb.no_batch || hipb.noalloc || hipb.sync_each || HB.flushing) return 0;
     if (gx == 0 || gy == 0 || (!solo && (u64)gx * gy > HB_MAX_BLOCKS) || (u64)gx * gy >= (1ull << 31) ||
         cf->threads == 0 || cf->threads % 64u ||
@@ -592,6 +736,7 @@ static int hb_hold(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *con
     h->ch_nb = 0;
     h->wg = 0;
     h->wmax = NULL;
+    h->row = row;
     h->hid = ++HB.next_hid;
     h->fn = fn;
     h->gx = gx;
@@ -606,14 +751,23 @@ static int hb_hold(const CoForm *cf, hipFunction_t fn, u32 gx, u32 gy, void *con
         off += cf->psz[j];
     }
     h->seq_start = 0;
+    if (!HB.n) HB.row = 0;
     const char *why = hb_joins(h);
     if (!why && HB.comb_used + comb_words > COMB_SLOTS) why = "combine area";
     if (!why && HB.seq && !hb_seq_join(h)) why = "sequence";
-    if (why && strcmp(why, "memory") == 0 && comb_param < 0 && hb_seq_join(h)) {
+    if (!HB.row && why && strcmp(why, "memory") == 0 && comb_param < 0 && hb_seq_join(h)) {
         /* depends on a held launch: the next step of a held sequence */
         h->seq_start = 1;
         HB.seq = 1;
         why = NULL;
+    }
+    if (HB.row || (why && HB.n && !HB.seq)) {
+        if (comb_param < 0 && !resident && hb_row_join(h)) {
+            HB.row = 1;
+            why = NULL;
+        } else if (HB.row) {
+            why = "rows";
+        }
     }
     if (why) {
         if (hipb.verbose && HB.n)
@@ -790,6 +944,7 @@ static int hb_set_launch(HbEnt *h, const CoForm *cf, hipFunction_t fn, u32 gx, u
     h->gy = gy;
     h->resident = resident;
     h->solo = 0;
+    h->row = NULL;
     return 1;
 }
 
@@ -998,6 +1153,7 @@ static int hb_try_epilogue(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, cons
 static void hb_release(void) {
     HB.n = 0;
     HB.seq = 0;
+    HB.row = 0;
     for (u32 i = 0; i < HB.ncache; i++) HIPB_CHECK(hipModuleUnload(HB.cache[i].mod));
     HB.ncache = 0;
 }
@@ -1687,9 +1843,10 @@ static void hb_run_generated(KCacheEntry *e, u32 out_buf, const u32 *leaf_bufs, 
     if (e->mode == KG_MODE_GROUP) grid_for(e->total, e->block, &gx, &gy);
     else grid_for((e->n_threads + e->block - 1) / e->block, e->block, &gx, &gy);
     /* a chainable program is held, alone if its grid is too large to
-     * batch, so that a consumer of its output can fuse after it */
-    if (hipb_hold(&e->co, e->fn, gx, gy, params, &hm, 0, -1, 0) ||
-        (e->chain && hb_hold_large(&e->co, e->fn, gx, gy, params, &hm)))
+     * batch, so that a consumer of its output can fuse after it, and a row
+     * reduction, so that programs on the same rows follow in its launch */
+    const int any = (e->chain || (e->row && !hipb.no_seq)) && !hipb.no_fuse;
+    if (hb_hold(&e->co, e->fn, gx, gy, params, &hm, 0, -1, 0, any ? 2 : 0, e->row))
         hb_hold_chain(e->chain, out_buf, leaf_bufs, n_leaves);
     else
         hipb_launch(e->fn, gx, gy, 1, e->block, params);
@@ -2182,6 +2339,57 @@ int thvm_hip_kernel_source(const UOpKernel *k, char *buf, u64 buflen, u32 *mode,
     if (vec) *vec = g.vec;
     kgen_free(&g);
     return (int)n;
+}
+
+/* Device-free: how a program takes each of its buffers (slot 0: the output)
+ * in a row sequence: 0 not at all, 1 matrix, 2 vector (div: gids of a row
+ * where it is elementwise), 3 otherwise. Returns the slots, 0 where it is no
+ * step of one. */
+int thvm_hip_row_classes(const UOpKernel *k, u32 *cls, u32 *div, u32 n) {
+    char err[256] = {0};
+    KGenResult g;
+    if (!kgen_uop(k, &g, err, sizeof err)) return 0;
+    RowInfo *ri = g.splits <= 1 ? row_info_make(k, g.mode == KG_MODE_GROUP, g.n_threads) : NULL;
+    kgen_free(&g);
+    int r = 0;
+    for (u32 s = 0; ri && s <= ri->n_leaves && s < n; s++, r++) {
+        cls[s] = ri->cls[s];
+        div[s] = ri->div[s];
+    }
+    free(ri);
+    return r;
+}
+
+/* Device-free check of the row sequence kernel of n programs in order: its
+ * source's code-object size, or -1 with the reason in errbuf. */
+int thvm_hip_row_compile_check(const UOpKernel *const *ks, u32 n, char *errbuf, u64 errlen) {
+    if (!ks || n == 0 || n > HB_MAX || !errbuf || errlen == 0) return -1;
+    HbEnt *ents = calloc(n, sizeof(HbEnt));
+    if (!ents) return -1;
+    int ok = 1;
+    for (u32 i = 0; i < n && ok; i++) {
+        KGenResult g;
+        ok = kgen_uop(ks[i], &g, errbuf, (size_t)errlen);
+        if (!ok) break;
+        ents[i].row = row_info_make(ks[i], g.mode == KG_MODE_GROUP, g.n_threads);
+        grid_for(g.mode == KG_MODE_GROUP ? g.total : (g.n_threads + g.block - 1) / g.block, g.block, &ents[i].gx, &ents[i].gy);
+        ok = g.splits <= 1 && co_form_make(&ents[i].co, g.src, g.name, g.block, NULL);
+        kgen_free(&g);
+    }
+    u32 m = 0, cols = 0, T = 0;
+    ok = ok && hb_row_shape(ents, n, &m, &cols, &T);
+    for (u32 i = 0; i < n && ok; i++) ok = hb_row_fits(&ents[i], m, cols, T);
+    long r = -1;
+    char *src = ok ? hb_row_source(ents, n, cols, T, "thvm_rows_check") : NULL;
+    if (src) r = rtc_compile_only(src, errbuf, (size_t)errlen);
+    else snprintf(errbuf, errlen, "no row sequence");
+    free(src);
+    for (u32 i = 0; i < n; i++) {
+        if (ents[i].co.src) co_form_free(&ents[i].co);
+        free((void *)ents[i].row);
+    }
+    free(ents);
+    return (int)r;
 }
 
 int thvm_hip_kernel_lanes(const UOpKernel *k, u32 *lanes, u32 n_words, u32 *mode, u32 *vec) {

@@ -1,6 +1,7 @@
 /*
  * chain.c - an elementwise program fused into the launch of the elementwise
- * program whose output it reads.
+ * program whose output it reads, and the programs that follow each other on
+ * the rows of one matrix.
  *
  * The engine dispatches each realized node as its own UOP_KERNEL
  * (src/schedule/_.c:2268-2411): batchnorm's normalisation and its scale and
@@ -223,4 +224,126 @@ int chain_merge(const ChainInfo *p, const u32 *pb, const UOpKernel *c, u32 c_out
     m->local_size = 0;
     m->out_dtype = p->out_dtype;
     return 1;
+}
+
+/* ---- programs that take a matrix row by row ----
+ *
+ * A softmax, its cross-entropy, a normalisation over rows are dispatched as
+ * reductions of each row and elementwise programs over the matrix, each
+ * reading what the ones before wrote (src/schedule/_.c:2268-2411). A program
+ * is recognised here when a buffer is read or written at the row of the
+ * output alone; held launches of such programs go out as one launch whose
+ * workgroups each take a row through all of them (backend.c, row sequences).
+ */
+
+/* Whether the part of `a` in x = gid (var 0) or the loop counter (var 1) is
+ * scale * (x / base); base 0: any, set to the one found. */
+static int is_scaled(const DCtx *c, const Aff *a, u8 var, u32 *base, u64 scale) {
+    u32 ord[DG_MAX], n = 0;
+    for (u32 t = 0; t < a->n; t++)
+        if (a->d[t].var == var) ord[n++] = t;
+    if (n == 0) return 0;
+    for (u32 i = 1; i < n; i++)
+        for (u32 j = i; j > 0 && a->d[ord[j - 1]].div > a->d[ord[j]].div; j--) {
+            const u32 x = ord[j];
+            ord[j] = ord[j - 1];
+            ord[j - 1] = x;
+        }
+    if (!*base) *base = a->d[ord[0]].div;
+    u64 step = *base;
+    for (u32 i = 0; i < n; i++) {
+        const Digit *d = &a->d[ord[i]];
+        if (d->div != step || step % *base || a->coef[ord[i]] != step / *base * scale) return 0;
+        if (i + 1 == n) return d->mod == 0 || (u64)d->div * d->mod >= var_range(c, var);
+        if (d->mod == 0) return 0;
+        step *= d->mod;
+        if (step > 0xFFFFFFFFull) return 0;
+    }
+    return 0;
+}
+
+static u32 vars(const Aff *a) {
+    u32 v = 0;
+    for (u32 t = 0; t < a->n; t++) v |= 1u << a->d[t].var;
+    return v;
+}
+
+static void note(RowInfo *ri, u32 slot, u8 cls, u32 div) {
+    if (ri->cls[slot] == ROW_UNUSED) {
+        ri->cls[slot] = cls;
+        ri->div[slot] = div;
+    } else if (ri->cls[slot] != cls || ri->div[slot] != div) {
+        ri->cls[slot] = ROW_OTHER;
+    }
+}
+
+RowInfo *row_info_make(const UOpKernel *k, int group, u64 n_threads) {
+    if (!k || k->n_leaves > FUSE_MAX_LEAVES || k->n_ops == 0 || k->n_ops > KOP_MAX) return NULL;
+    const u32 total = launch_total(k);
+    i32 loop = -1;
+    u32 loops = 0, depth = 0;
+    if (total < 2) return NULL;
+    for (u32 i = 0; i < k->n_ops; i++) {
+        const KOpType t = k->ops[i].type;
+        if (t == KOP_RANGE) {
+            loop = (i32)i;
+            loops++;
+            depth++;
+        } else if (t == KOP_ENDRANGE) {
+            if (depth-- == 0) return NULL;
+        } else if (t == KOP_STORE && (depth || k->ops[i].imm.u > k->n_leaves)) {
+            return NULL;
+        }
+    }
+    if (loops != (group ? 1u : 0u)) return NULL;
+    const u32 trip = group ? k->ops[loop].imm.u : 0;
+    if (group && (trip < 2 || (u64)total * trip > 0xFFFFFFFFull)) return NULL;
+    Aff *aff = calloc(k->n_ops, sizeof(Aff));
+    RowInfo *ri = calloc(1, sizeof *ri);
+    int ok = aff && ri;
+    if (ok) {
+        DCtx dc = {k, total, group ? trip : 1, loop, aff};
+        analyze_aff(&dc);
+        ri->total = total;
+        ri->trip = trip;
+        ri->n_leaves = k->n_leaves;
+        ri->per = !group && n_threads && total % n_threads == 0 ? (u32)(total / n_threads) : 0;
+        for (u32 i = 0; i < k->n_ops && ok; i++) {
+            const KOp *op = &k->ops[i];
+            if (op->type != KOP_LOAD && op->type != KOP_STORE) continue;
+            const u32 slot = op->imm.u;
+            if (slot > k->n_leaves) continue;   /* reads no buffer */
+            const Aff *a = &aff[op->arg[0]];
+            u32 one = 1, base = 0;
+            u8 cls = ROW_OTHER;
+            if (!a->ok || a->cst || a->n == 0 || a->n > DG_MAX) {
+                ;
+            } else if (aff_is_gid(&dc, a)) {
+                cls = group ? ROW_VECTOR : ROW_MATRIX;
+            } else if (group) {
+                if (is_scaled(&dc, a, 0, &one, trip) && is_scaled(&dc, a, 1, &one, 1)) cls = ROW_MATRIX;
+            } else if (vars(a) == 1u && is_scaled(&dc, a, 0, &base, 1)) {
+                cls = ROW_VECTOR;
+            }
+            if (op->type == KOP_STORE) {
+                ok = aff_is_gid(&dc, a);
+                ri->writes |= slot < 64 ? 1ull << slot : 0;
+                ok = ok && slot < 64;
+            }
+            note(ri, slot, cls, cls == ROW_VECTOR && !group ? base : 0);
+        }
+        for (u32 s = 0; s <= k->n_leaves; s++) ri->f16[s] = (s ? k->leaf_dtypes[s - 1] : k->out_dtype) == DTYPE_F16;
+    }
+    free(aff);
+    if (!ok) {
+        free(ri);
+        return NULL;
+    }
+    return ri;
+}
+
+int row_slots_agree(const RowInfo *a, u32 sa, const RowInfo *b, u32 sb, u32 n) {
+    if (a->cls[sa] != b->cls[sb] || (a->cls[sa] != ROW_MATRIX && a->cls[sa] != ROW_VECTOR) || a->f16[sa] != b->f16[sb]) return 0;
+    if (a->cls[sa] == ROW_MATRIX) return 1;
+    return (a->trip || a->div[sa] == n) && (b->trip || b->div[sb] == n);
 }

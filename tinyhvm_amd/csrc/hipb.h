@@ -268,6 +268,7 @@ typedef struct {
     u32 np;
     u8 psz[CO_MAX_PARAMS]; /* its parameters' sizes in bytes */
     u8 no_sync;            /* no workgroup barrier or LDS of its own */
+    u8 lane_free;          /* ... and no exchange between lanes: any lane may run as any other */
 } CoForm;
 int  co_form_make(CoForm *cf, const char *src, const char *name, u32 threads, hipFunction_t fn);
 void co_form_free(CoForm *cf);
@@ -330,6 +331,27 @@ int chain_merge(const ChainInfo *p, const u32 *pb, const UOpKernel *c, u32 c_out
 /* bit s set: the program STOREs into leaf slot s (s >= 1) */
 u64 chain_store_slots(const UOpKernel *k);
 
+/* ---------------- rows (chain.c) ---------------- */
+/* How a program over [m, n] takes its buffers: a reduction of each row into
+ * one output (total = m, trip = n), or an elementwise program (total = m n).
+ * A buffer is a matrix (element i n + j at row i, column j), a vector
+ * (element i at row i), or neither. */
+enum { ROW_UNUSED = 0, ROW_MATRIX, ROW_VECTOR, ROW_OTHER };
+typedef struct {
+    u32 total, trip;          /* trip 0: elementwise */
+    u32 per;                  /* elementwise: gids of a thread (0: its threads do not divide them evenly) */
+    u32 n_leaves;
+    u64 writes;               /* bit s: slot s is stored to (0: the output) */
+    u8 cls[FUSE_MAX_LEAVES + 1], f16[FUSE_MAX_LEAVES + 1];
+    u32 div[FUSE_MAX_LEAVES + 1];   /* an elementwise program's vector: at gid / div */
+} RowInfo;
+/* The row form of a program generated as `group` (a workgroup an output) or
+ * with n_threads threads, or NULL. */
+RowInfo *row_info_make(const UOpKernel *k, int group, u64 n_threads);
+/* Whether a's and b's slots sa and sb, on the same buffer, touch only the
+ * same row of it in each row of [m, n]. */
+int row_slots_agree(const RowInfo *a, u32 sa, const RowInfo *b, u32 sb, u32 n);
+
 /* ---------------- rtc / cache ---------------- */
 typedef struct {
     u64 key;
@@ -347,6 +369,7 @@ typedef struct {
     char name[32];        /* the kernel's symbol */
     CoForm co;            /* its co-launch form */
     ChainInfo *chain;     /* set when a consumer may fuse after it */
+    RowInfo *row;         /* set when it may be a step of a row sequence */
     u64 store_slots;      /* leaf slots it writes (chain_store_slots) */
 } KCacheEntry;
 

@@ -105,6 +105,7 @@ void rtc_shutdown(void) {
                 HIPB_CHECK(hipModuleUnload(R.tab[i].mod));
                 free(R.tab[i].ops);
                 free(R.tab[i].chain);
+                free(R.tab[i].row);
                 co_form_free(&R.tab[i].co);
             }
         }
@@ -435,6 +436,8 @@ int co_form_make(CoForm *cf, const char *src, const char *name, u32 threads, hip
     cf->threads = threads;
     cf->no_sync = !strstr(o, "__syncthreads") && !strstr(o, "bsum_n<") && !strstr(o, "bmax_n<") &&
                   !strstr(o, "__shared__");
+    cf->lane_free = cf->no_sync && !strstr(o, "__shfl") && !strstr(o, "__ballot") && !strstr(o, "readfirstlane") &&
+                    !strstr(o, "wsum") && !strstr(o, "wmax");
     if (fn) {   /* NULL: a device-free check */
         int v = 0;
         if (hipFuncGetAttribute(&v, HIP_FUNC_ATTRIBUTE_SHARED_SIZE_BYTES, fn) != hipSuccess || v < 0) goto fail_src;
@@ -537,6 +540,7 @@ again:
     if (!g.combine_launch) co_form_make(&e->co, g.src, g.name, g.block, fn);
     e->store_slots = chain_store_slots(k);
     e->chain = (e->ops && g.mode != KG_MODE_GROUP && g.splits <= 1) ? chain_info_make(k, e->ops) : NULL;
+    e->row = g.splits <= 1 ? row_info_make(k, g.mode == KG_MODE_GROUP, g.n_threads) : NULL;
     hipb.n_compile++;
     kgen_free(&g);
     return e;
