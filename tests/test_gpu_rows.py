@@ -72,7 +72,7 @@ def run(m, n, data):
     return outs
 
 
-@pytest.mark.parametrize("m,n", [(2, 256), (65, 260), (64, 1000), (33, 1001), (700, 1024), (4096, 1000), (2100, 5000), (300, 5000)])
+@pytest.mark.parametrize("m,n", [(2, 256), (65, 260), (64, 1000), (33, 1001), (700, 1024), (4096, 1000), (2100, 5000), (300, 8192), (40, 8196)])
 def test_rows_as_separate_launches(m, n, monkeypatch):
     rng = np.random.default_rng(m * 7 + n)
     f = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731

@@ -119,10 +119,11 @@ static void copyq_guard_dispatch(u32 out, const u32 *leaves, u32 n) {
  * the launches left: the cross-entropy head over [4096, 1000] (nine launches,
  * 52.0 us) is four, 30.7 us (the first three reductions 10.6 us, maxima to
  * gradient 17.3), a fused chain and its gradient over [8192, 8192], whose
- * rows do not stay in the L2, 290 -> 276 us. A long row needs enough of them to fill the GPU:
- * rows of more than HB_ROW_LONG elements join from HB_ROW_MANY of them. */
-#define HB_ROW_LONG 4096u
-#define HB_ROW_MANY 2048u
+ * rows do not stay in the L2, 290 -> 276 us. Over rows of 8192 the head
+ * gains while the matrix fits the last cache (600 rows 58.5 -> 40.6 us, 1500
+ * 104 -> 92, 2048 133 -> 129) and loses where it does not (3000 rows 188 ->
+ * 192); longer rows stay launches of their own. */
+#define HB_ROW_LONG 8192u
 #define HB_SEQ_MAX_BLOCKS 4u
 #define HB_SEQ_THREADS 256u
 #define HB_MAX 16
@@ -660,7 +661,7 @@ static int hb_row_join(const HbEnt *h) {
     u32 m, cols, T;
     if (HB.n == 0 || HB.n >= HB_MAX) return 0;
     if (!hb_row_shape(HB.ent, HB.n, &m, &cols, &T) && !hb_row_shape(h, 1, &m, &cols, &T)) return 0;
-    if (!hb_row_fits(h, m, cols, T) || (cols > HB_ROW_LONG && m < HB_ROW_MANY)) return 0;
+    if (!hb_row_fits(h, m, cols, T) || cols > HB_ROW_LONG) return 0;
     u32 lds = h->co.lds;
     int gain = 0;
     for (u32 i = 0; i < HB.n; i++) {
