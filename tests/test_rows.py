@@ -52,3 +52,16 @@ def test_softmax_compiles_as_one_kernel():
     with pytest.raises(ValueError):   # a thread's four elements cross the row's end
         _lib.row_compile_check([rp.program(64, 1001, [MAT], lambda o, v: v, reduce=RMAX),
                                 rp.program(64, 1001, [MAT], lambda o, v: o(abi.UOP_EXP, v))])
+
+
+def test_a_thread_of_pieces_of_two_rows_is_no_step(monkeypatch):
+    """With several vectors a thread, a thread's elements lie far apart: a
+    workgroup's threads would reach rows that other workgroups still reduce."""
+    ks = [rp.program(4096, 1000, [MAT], lambda o, v: v, reduce=RMAX),
+          rp.program(4096, 1000, [MAT, VEC], lambda o, a, b: o(abi.UOP_EXP, o(abi.UOP_SUB, a, b)))]
+    assert _lib.row_compile_check(ks) > 0
+    for per in "28":
+        monkeypatch.setenv("THVM_HIP_EW_PER_THREAD", per)
+        assert "w_ < %su" % per in _lib.kernel_source(ks[1])[0]
+        with pytest.raises(ValueError):
+            _lib.row_compile_check(ks)

@@ -2350,7 +2350,7 @@ int thvm_hip_row_classes(const UOpKernel *k, u32 *cls, u32 *div, u32 n) {
     char err[256] = {0};
     KGenResult g;
     if (!kgen_uop(k, &g, err, sizeof err)) return 0;
-    RowInfo *ri = g.splits <= 1 ? row_info_make(k, g.mode == KG_MODE_GROUP, g.n_threads) : NULL;
+    RowInfo *ri = g.splits <= 1 ? row_info_make(k, g.mode == KG_MODE_GROUP, g.per) : NULL;
     kgen_free(&g);
     int r = 0;
     for (u32 s = 0; ri && s <= ri->n_leaves && s < n; s++, r++) {
@@ -2372,7 +2372,7 @@ int thvm_hip_row_compile_check(const UOpKernel *const *ks, u32 n, char *errbuf, 
         KGenResult g;
         ok = kgen_uop(ks[i], &g, errbuf, (size_t)errlen);
         if (!ok) break;
-        ents[i].row = row_info_make(ks[i], g.mode == KG_MODE_GROUP, g.n_threads);
+        ents[i].row = row_info_make(ks[i], g.mode == KG_MODE_GROUP, g.per);
         grid_for(g.mode == KG_MODE_GROUP ? g.total : (g.n_threads + g.block - 1) / g.block, g.block, &ents[i].gx, &ents[i].gy);
         ok = g.splits <= 1 && co_form_make(&ents[i].co, g.src, g.name, g.block, NULL);
         kgen_free(&g);

@@ -277,7 +277,7 @@ static void note(RowInfo *ri, u32 slot, u8 cls, u32 div) {
     }
 }
 
-RowInfo *row_info_make(const UOpKernel *k, int group, u64 n_threads) {
+RowInfo *row_info_make(const UOpKernel *k, int group, u32 per) {
     if (!k || k->n_leaves > FUSE_MAX_LEAVES || k->n_ops == 0 || k->n_ops > KOP_MAX) return NULL;
     const u32 total = launch_total(k);
     i32 loop = -1;
@@ -307,7 +307,7 @@ RowInfo *row_info_make(const UOpKernel *k, int group, u64 n_threads) {
         ri->total = total;
         ri->trip = trip;
         ri->n_leaves = k->n_leaves;
-        ri->per = !group && n_threads && total % n_threads == 0 ? (u32)(total / n_threads) : 0;
+        ri->per = group ? 0 : per;
         for (u32 i = 0; i < k->n_ops && ok; i++) {
             const KOp *op = &k->ops[i];
             if (op->type != KOP_LOAD && op->type != KOP_STORE) continue;

@@ -204,6 +204,7 @@ typedef struct {
     u32 block;            /* threads per workgroup */
     u64 total;            /* serial: gids; group: outputs */
     u64 n_threads;        /* serial: number of vector lanes (ceil(total/vec)) */
+    u32 per;              /* serial: thread t takes gids [t * per, (t + 1) * per) (0: others as well) */
     u32 splits;           /* group: workgroups per output (> 1: partials combined in one pass) */
     int combine_launch;   /* ... or, with splits > 1, by a separate <name>_fin kernel */
     u32 n_scal;           /* constant-index leaf loads that take an inline value (sm_, sv*) */
@@ -339,15 +340,16 @@ u64 chain_store_slots(const UOpKernel *k);
 enum { ROW_UNUSED = 0, ROW_MATRIX, ROW_VECTOR, ROW_OTHER };
 typedef struct {
     u32 total, trip;          /* trip 0: elementwise */
-    u32 per;                  /* elementwise: gids of a thread (0: its threads do not divide them evenly) */
+    u32 per;                  /* elementwise: consecutive gids of a thread (0: they are further apart) */
     u32 n_leaves;
     u64 writes;               /* bit s: slot s is stored to (0: the output) */
     u8 cls[FUSE_MAX_LEAVES + 1], f16[FUSE_MAX_LEAVES + 1];
     u32 div[FUSE_MAX_LEAVES + 1];   /* an elementwise program's vector: at gid / div */
 } RowInfo;
 /* The row form of a program generated as `group` (a workgroup an output) or
- * with n_threads threads, or NULL. */
-RowInfo *row_info_make(const UOpKernel *k, int group, u64 n_threads);
+ * with threads of `per` consecutive gids each (0: of gids further apart), or
+ * NULL. */
+RowInfo *row_info_make(const UOpKernel *k, int group, u32 per);
 /* Whether a's and b's slots sa and sb, on the same buffer, touch only the
  * same row of it in each row of [m, n]. */
 int row_slots_agree(const RowInfo *a, u32 sa, const RowInfo *b, u32 sb, u32 n);

@@ -1786,6 +1786,7 @@ int kgen_uop_lanes(const UOpKernel *k, KGenResult *out, u32 *lanes, char *err, s
         emit_range_seq(&G, 0, k->n_ops, 0, 0);
         if (W > 1) sb_put(s, "  }\n");
         out->n_threads = nthreads;
+        out->per = W == 1 ? G.V : 0;
     } else {
         if (G.splits > 1) {
             sb_put(s, "  const u32 bid_ = blockIdx.y * gridDim.x + blockIdx.x;\n");

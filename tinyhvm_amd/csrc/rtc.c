@@ -540,7 +540,7 @@ again:
     if (!g.combine_launch) co_form_make(&e->co, g.src, g.name, g.block, fn);
     e->store_slots = chain_store_slots(k);
     e->chain = (e->ops && g.mode != KG_MODE_GROUP && g.splits <= 1) ? chain_info_make(k, e->ops) : NULL;
-    e->row = g.splits <= 1 ? row_info_make(k, g.mode == KG_MODE_GROUP, g.n_threads) : NULL;
+    e->row = g.splits <= 1 ? row_info_make(k, g.mode == KG_MODE_GROUP, g.per) : NULL;
     hipb.n_compile++;
     kgen_free(&g);
     return e;
