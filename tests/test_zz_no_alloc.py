@@ -28,6 +28,7 @@ import os
 import numpy as np
 import pytest
 
+from tests import contractions
 from tests import tracetools as tt
 from tests.test_gpu_parity import _reads_own_output
 from tinyhvm_amd import _lib, trace
@@ -232,5 +233,40 @@ def test_noalloc_after_fused_step():
         assert n >= 50
         n = _fused_then_noalloc(L, os.path.join(WL, "mlp_64x784x128x10.trc"), "mlp.fwd", None)
         assert n >= 15
+    finally:
+        _restore(L, saved)
+
+
+@pytest.mark.parametrize("m,k,n", [(2048, 2048, 2048), (1024, 4096, 2048), (4096, 1024, 1024)], ids=lambda v: str(v))
+def test_partial_sums_that_fill_the_workspace(m, k, n):
+    """Contractions whose f32 split-K partials are exactly the static
+    workspace: the marks of the plane tile ahead of them lie behind it. One
+    element is infinite, so that some tiles take the f32 kernel."""
+    L, saved = _fresh({})
+    try:
+        prog, sa, sb = contractions.matmul("nn", m, k, n)
+        assert "redo_(" in _lib.dense_source(prog)
+        a = _lib.dense_analyze(prog)
+        assert a[3] * m * n * 4 == 32 << 20, a
+        rng = np.random.default_rng(m + k)
+        xs = [rng.uniform(-1, 1, s).astype(np.float32) for s in (sa, sb)]
+        xs[0][3, 5] = np.inf
+        ids = []
+        for x in xs:
+            ids.append(L.thvm_hip_buf_alloc(x.nbytes))
+            L.thvm_hip_buf_write(ids[-1], x.ctypes.data_as(C.c_void_p), x.nbytes)
+        out = L.thvm_hip_buf_alloc(4 * m * n)
+        leaves = (C.c_uint32 * 2)(*ids)
+        L.thvm_hip_dispatch_uop_kernel(out, leaves, 2, C.byref(prog), 0)
+        want = _read(L, out, 4 * m * n)
+        fill = np.full_like(want, SENTINEL)
+        L.thvm_hip_buf_write(out, fill.ctypes.data_as(C.c_void_p), 4 * m * n)
+        assert L.thvm_hip_synchronize() == 0
+        c0 = _counters(L)
+        assert L.thvm_hip_dispatch_uop_kernel_noalloc(out, leaves, 2, C.byref(prog)) == OK
+        c1 = _counters(L)
+        assert c1[7] == c0[7] and c1[2] == c0[2]
+        assert np.array_equal(_read(L, out, 4 * m * n), want)
+        assert L.thvm_hip_synchronize() == 0
     finally:
         _restore(L, saved)

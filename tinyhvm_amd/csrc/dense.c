@@ -3421,7 +3421,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         if (!ws) return 0;
     }
     if (pt) {
-        fl = scratch_reserve(&D.fl, (u64)pt->tiles_m * pt->tiles_n * pt->splits * sizeof(u32));
+        fl = scratch_marks(&D.fl, (u64)pt->tiles_m * pt->tiles_n * pt->splits * sizeof(u32));
         if (!fl) return 0;
     }
     /* packed B side */

@@ -173,6 +173,7 @@ typedef struct { void *ptr; u64 cap; } Scratch;
 void *pool_block_get(u64 bytes, u64 *cap_out);
 void  pool_block_put(void *ptr, u64 cap);
 void *scratch_reserve(Scratch *sc, u64 bytes);
+void *scratch_marks(Scratch *sc, u64 bytes);
 void  scratch_release(Scratch *sc);
 void  pool_upload(void *dst, const void *src, u64 bytes);
 void  pool_free(u32 id);

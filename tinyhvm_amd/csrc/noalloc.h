@@ -8,7 +8,11 @@
 
 #include "thvm_hip.h"
 
-/* bytes of the array on each GPU: THVM_HIP_NOALLOC_SCRATCH_BYTES (thvm_hip.h) */
+/* bytes of the array on each GPU: THVM_HIP_NOALLOC_SCRATCH_BYTES (thvm_hip.h)
+ * of workspaces and, behind them, these for the marks of a plane tile's tiles
+ * (dense.c): partial sums that fill the workspaces exactly, as those of
+ * 2048x2048x2048 do, still leave the marks their place */
+#define THVM_NOALLOC_MARK_BYTES (64u << 10)
 #define THVM_NOALLOC_MAX_DEVICES 64
 
 #ifdef __cplusplus

@@ -14,7 +14,7 @@
 
 #include "noalloc.h"
 
-static __device__ __align__(256) unsigned char scratch[THVM_HIP_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[THVM_HIP_NOALLOC_SCRATCH_BYTES + THVM_NOALLOC_MARK_BYTES];
 
 static void *scratch_dev[THVM_NOALLOC_MAX_DEVICES];
 

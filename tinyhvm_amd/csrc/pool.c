@@ -42,6 +42,7 @@
 #include <string.h>
 
 #include "hipb.h"
+#include "noalloc.h"
 #include "thvm_hip.h"
 
 #define POOL_MIN_CLASS_BYTES 256ull
@@ -271,7 +272,7 @@ static void *noalloc_carve(u64 bytes) {
 
 static int in_static_scratch(const void *p) {
     const u8 *s = hipb.noalloc_scratch;
-    return s && (const u8 *)p >= s && (const u8 *)p < s + THVM_HIP_NOALLOC_SCRATCH_BYTES;
+    return s && (const u8 *)p >= s && (const u8 *)p < s + THVM_HIP_NOALLOC_SCRATCH_BYTES + THVM_NOALLOC_MARK_BYTES;
 }
 
 /* A released block: to limbo while a graph references it, else to its
@@ -459,6 +460,14 @@ void *scratch_reserve(Scratch *sc, u64 bytes) {
     sc->ptr = pool_block_get(bytes, &sc->cap);
     if (!sc->ptr) sc->cap = 0;
     return sc->ptr;
+}
+
+/* The same for a plane tile's marks: without allocation they lie behind the
+ * other workspaces, so that they take none of their room. */
+void *scratch_marks(Scratch *sc, u64 bytes) {
+    if (hipb.noalloc && hipb.noalloc_scratch && bytes <= THVM_NOALLOC_MARK_BYTES)
+        return (u8 *)hipb.noalloc_scratch + THVM_HIP_NOALLOC_SCRATCH_BYTES;
+    return scratch_reserve(sc, bytes);
 }
 
 void scratch_release(Scratch *sc) {
