@@ -94,3 +94,38 @@ def test_rows_as_separate_launches(m, n, monkeypatch):
         # exp's own error, the difference's and n additions', each within 2^-24 of a term
         err = np.abs(got["p"] - e / e.sum(1, keepdims=True)) / (e / e.sum(1, keepdims=True))
         assert err.max() <= (n + 64) * 2.0 ** -24
+
+
+def test_passes_are_the_same_kernels_however_many_run_on(monkeypatch):
+    """A pass over one matrix, dispatched 1 to 9 times before its launches go
+    out: the kernels of the first passes serve all of them."""
+    m, n = 300, 512
+    st = [("e", ["x", "c"], rp.program(m, n, [MAT, COL], two(MUL))), ("s", ["e"], rp.program(m, n, [MAT], one, reduce=SUM)),
+          ("p", ["e", "s"], rp.program(m, n, [MAT, VEC], two(SUB)))]
+    L = _lib.lib()
+    L.thvm_hip_shutdown()
+    assert L.thvm_hip_init() == 0
+    rng = np.random.default_rng(3)
+    data = {k: rng.standard_normal(s).astype(np.float32) for k, s in (("x", (m, n)), ("c", n), ("e", (m, n)), ("s", m), ("p", (m, n)))}
+    ids = {}
+    for k, v in data.items():
+        ids[k] = L.thvm_hip_buf_alloc(v.nbytes)
+        L.thvm_hip_buf_write(ids[k], v.ctypes.data_as(C.c_void_p), v.nbytes)
+
+    def passes(count):
+        for _ in range(count):
+            for out, leaves, k in st:
+                L.thvm_hip_dispatch_uop_kernel(ids[out], (C.c_uint32 * len(leaves))(*[ids[q] for q in leaves]), len(leaves), C.byref(k), 0)
+        assert L.thvm_hip_synchronize() == 0
+        c, p = (C.c_uint64 * 16)(), np.empty_like(data["p"])
+        L.thvm_hip_counters(c, 16)
+        L.thvm_hip_buf_read(ids["p"], p.ctypes.data_as(C.c_void_p), p.nbytes)
+        return c[2], c[11], p
+
+    compiled, batched, want = passes(2)
+    for count in (1, 3, 4, 6, 9):
+        c, b, p = passes(count)
+        assert c == compiled and b - batched == 3 * count, count    # the three launches of a pass in one
+        assert p.tobytes() == want.tobytes()
+        batched = b
+    L.thvm_hip_shutdown()

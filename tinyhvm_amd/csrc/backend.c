@@ -115,7 +115,12 @@ static void copyq_guard_dispatch(u32 out, const u32 *leaves, u32 n) {
  * are not streamed past the caches. Every program's code is its own device
  * function, an elementwise one called for the row's threads with the block
  * and lane each has in its own launch: the results are those of separate
- * launches bit for bit. Bound by the rows' bytes through the XCD's cache and
+ * launches bit for bit. A sequence ends where a program that it holds comes
+ * again: a pass dispatched over and over is then the same kernels however
+ * many times it runs before something issues them (without that rule the
+ * passes joined up to HB_MAX launches, every number of them a kernel to
+ * compile: 20 passes of the fused chain over [8192, 8192] took 23 ms each).
+ * Bound by the rows' bytes through the XCD's cache and
  * the launches left: the cross-entropy head over [4096, 1000] (nine launches,
  * 52.0 us) is four, 30.7 us (the first three reductions 10.6 us, maxima to
  * gradient 17.3), a fused chain and its gradient over [8192, 8192], whose
@@ -162,8 +167,14 @@ static struct {
     int flushing;
     int seq;               /* the held launches are a sequence of dependent steps (hb_seq_*) */
     int row;               /* ... a row sequence (hb_row_*) */
-    struct { u64 key; hipModule_t mod; hipFunction_t fn; u32 cap; } cache[64];
-    u32 ncache;
+    /* the kernels built for sets of held launches; row sequences have a table
+     * of their own, so that however many of them a process meets, its batches
+     * and sequences find theirs. Kernels stay loaded until shutdown: a graph
+     * may hold any of them. */
+    struct {
+        struct { u64 key; hipModule_t mod; hipFunction_t fn; u32 cap; } e[64];
+        u32 n;
+    } cache[2];
 } HB;
 
 static int hb_seq_eligible(const HbEnt *h);
@@ -363,12 +374,14 @@ static char *hb_batch_source(const HbEnt *ents, u32 n, u32 T, const char *name) 
  * workgroups of it the GPU holds at once (*cap). */
 static hipFunction_t hb_batch_fn(u64 key, u32 T, u32 *cap, int seq) {   /* seq 2: a row sequence */
     *cap = 0;
-    for (u32 i = 0; i < HB.ncache; i++)
-        if (HB.cache[i].key == key) {
-            *cap = HB.cache[i].cap;
-            return HB.cache[i].fn;
+    const int tab = seq == 2;
+    u32 *nc = &HB.cache[tab].n;
+    for (u32 i = 0; i < *nc; i++)
+        if (HB.cache[tab].e[i].key == key) {
+            *cap = HB.cache[tab].e[i].cap;
+            return HB.cache[tab].e[i].fn;
         }
-    if (HB.ncache >= sizeof HB.cache / sizeof HB.cache[0]) return NULL;
+    if (*nc >= sizeof HB.cache[tab].e / sizeof HB.cache[tab].e[0]) return NULL;
     char name[48];
     snprintf(name, sizeof name, "thvm_%s_%016llx", seq == 2 ? "rows" : seq ? "seq" : "batch", (unsigned long long)key);
     u32 m, cols, rt;
@@ -388,11 +401,11 @@ static hipFunction_t hb_batch_fn(u64 key, u32 T, u32 *cap, int seq) {   /* seq 2
     hipFunction_t fn = NULL;
     if (rtc_build_module(src, &mod, err, sizeof err)) {
         if (hipModuleGetFunction(&fn, mod, name) == hipSuccess) {
-            HB.cache[HB.ncache].key = key;
-            HB.cache[HB.ncache].mod = mod;
-            HB.cache[HB.ncache].fn = fn;
-            HB.cache[HB.ncache].cap = *cap = rtc_capacity(fn, T);
-            HB.ncache++;
+            HB.cache[tab].e[*nc].key = key;
+            HB.cache[tab].e[*nc].mod = mod;
+            HB.cache[tab].e[*nc].fn = fn;
+            HB.cache[tab].e[*nc].cap = *cap = rtc_capacity(fn, T);
+            (*nc)++;
             hipb.n_compile++;
         } else {
             HIPB_CHECK(hipModuleUnload(mod));
@@ -665,6 +678,7 @@ static int hb_row_join(const HbEnt *h) {
     u32 lds = h->co.lds;
     int gain = 0;
     for (u32 i = 0; i < HB.n; i++) {
+        if (HB.ent[i].co.id == h->co.id) return 0;    /* the next pass begins */
         if (!hb_row_fits(&HB.ent[i], m, cols, T) || !hb_row_pair(&HB.ent[i], h, cols, &gain)) return 0;
         lds += HB.ent[i].co.lds;
     }
@@ -1155,8 +1169,10 @@ static void hb_release(void) {
     HB.n = 0;
     HB.seq = 0;
     HB.row = 0;
-    for (u32 i = 0; i < HB.ncache; i++) HIPB_CHECK(hipModuleUnload(HB.cache[i].mod));
-    HB.ncache = 0;
+    for (u32 t = 0; t < 2; t++) {
+        for (u32 i = 0; i < HB.cache[t].n; i++) HIPB_CHECK(hipModuleUnload(HB.cache[t].e[i].mod));
+        HB.cache[t].n = 0;
+    }
 }
 
 static int env_flag(const char *name) {
