@@ -129,3 +129,33 @@ def test_passes_are_the_same_kernels_however_many_run_on(monkeypatch):
         assert p.tobytes() == want.tobytes()
         batched = b
     L.thvm_hip_shutdown()
+
+
+@pytest.mark.parametrize("m,n,rows", [(2, 4092, True), (64, 4096, False), (64, 8192, False), (256, 4096, True), (300, 8192, True), (300, 8196, False)],
+                         ids=str)
+def test_which_rows_are_a_sequence(m, n, rows):
+    st = [("e", ["x", "c"], rp.program(m, n, [MAT, COL], two(MUL))), ("s", ["e"], rp.program(m, n, [MAT], one, reduce=RMAX)),
+          ("p", ["e", "s"], rp.program(m, n, [MAT, VEC], two(SUB)))]
+    L = _lib.lib()
+    L.thvm_hip_shutdown()
+    assert L.thvm_hip_init() == 0
+    x = np.random.default_rng(m + n).standard_normal((m, n)).astype(np.float32)
+    c = np.linspace(0.5, 2, n, dtype=np.float32)
+    ids = {k: L.thvm_hip_buf_alloc(4 * m * n) for k in "xep"}
+    ids.update(c=L.thvm_hip_buf_alloc(4 * n), s=L.thvm_hip_buf_alloc(4 * m))
+    for k, v in (("x", x), ("c", c)):
+        L.thvm_hip_buf_write(ids[k], v.ctypes.data_as(C.c_void_p), v.nbytes)
+    batched = []
+    for _ in range(2):
+        for out, leaves, k in st:
+            L.thvm_hip_dispatch_uop_kernel(ids[out], (C.c_uint32 * len(leaves))(*[ids[q] for q in leaves]), len(leaves), C.byref(k), 0)
+        assert L.thvm_hip_synchronize() == 0
+        cnt = (C.c_uint64 * 16)()
+        L.thvm_hip_counters(cnt, 16)
+        batched.append(cnt[11])
+    assert batched[1] - batched[0] == (3 if rows else 0)
+    p = np.empty_like(x)
+    L.thvm_hip_buf_read(ids["p"], p.ctypes.data_as(C.c_void_p), p.nbytes)
+    e = x * c
+    assert np.array_equal(p, e - e.max(1, keepdims=True))
+    L.thvm_hip_shutdown()

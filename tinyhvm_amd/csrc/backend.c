@@ -120,14 +120,25 @@ static void copyq_guard_dispatch(u32 out, const u32 *leaves, u32 n) {
  * many times it runs before something issues them (without that rule the
  * passes joined up to HB_MAX launches, every number of them a kernel to
  * compile: 20 passes of the fused chain over [8192, 8192] took 23 ms each).
- * Bound by the rows' bytes through the XCD's cache and
- * the launches left: the cross-entropy head over [4096, 1000] (nine launches,
- * 52.0 us) is four, 30.7 us (the first three reductions 10.6 us, maxima to
- * gradient 17.3), a fused chain and its gradient over [8192, 8192], whose
- * rows do not stay in the L2, 290 -> 276 us. Over rows of 8192 the head
- * gains while the matrix fits the last cache (600 rows 58.5 -> 40.6 us, 1500
- * 104 -> 92, 2048 133 -> 129) and loses where it does not (3000 rows 188 ->
- * 192); longer rows stay launches of their own. */
+ * Bound by the rows' bytes through the XCD's cache and the launches left: the
+ * cross-entropy head over [4096, 1000] (nine launches, 52.0 us) is four, 30.7
+ * us (the first three reductions 10.6 us, maxima to gradient 17.3).
+ *
+ * Which rows, in us as a sequence / as separate launches, on the same buffers
+ * each pass and on three sets in turn. Rows longer than 8192 stay separate:
+ * what a workgroup reads again has left the caches by then, and a matrix is
+ * read less evenly (a fused chain and its gradient over rows of 8192: 8192
+ * of them 271 / 271 and 274 / 289, 3000 104 / 104 and 107 / 109, 600 21 / 25
+ * and 21 / 26; of 10240: 3000 144 / 128 and 143 / 137; of 16384: 4096 350 /
+ * 272 and 350 / 291; the cross-entropy head over rows of 8192: 8192 of them
+ * 477 / 501 on both, 3000 192 / 189 and 191 / 201, 600 41 / 58 and 43 / 58).
+ * The engine's own chain over [8192, 8192], on the same buffers, is the one
+ * that loses: 280 / 274. Long rows need a row for each compute unit, or the
+ * elementwise programs, whose own launches have a workgroup for every few KB
+ * of a row, leave units idle (the head over 64 rows of 8192 26.8 / 25.8 and
+ * 28.7 / 25.7, 2 of 4096 26.7 / 25.9 and 29.1 / 25.5, 256 of 4096 26.7 /
+ * 26.8; 2 of 3072, whose sums are steps too, 18 / 28). */
+#define HB_ROW_WIDE 4096u
 #define HB_ROW_LONG 8192u
 #define HB_SEQ_MAX_BLOCKS 4u
 #define HB_SEQ_THREADS 256u
@@ -675,6 +686,7 @@ static int hb_row_join(const HbEnt *h) {
     if (HB.n == 0 || HB.n >= HB_MAX) return 0;
     if (!hb_row_shape(HB.ent, HB.n, &m, &cols, &T) && !hb_row_shape(h, 1, &m, &cols, &T)) return 0;
     if (!hb_row_fits(h, m, cols, T) || cols > HB_ROW_LONG) return 0;
+    if (cols >= HB_ROW_WIDE && m < (hipb.n_cu ? hipb.n_cu : 256u)) return 0;
     u32 lds = h->co.lds;
     int gain = 0;
     for (u32 i = 0; i < HB.n; i++) {
