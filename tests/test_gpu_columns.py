@@ -104,3 +104,21 @@ def test_column_sums(m, n, kind, dt):
     bound = (m / 64 + 32 + 1) * 2.0 ** -24 * mag + (np.abs(want) * 2.0 ** -11 + 2.0 ** -25 if dt == F16 else 0)
     worst = np.max(np.abs(out.astype(np.float64) - want) / bound)
     assert worst <= 1.0, worst
+
+
+# fewer columns a workgroup where the grid is small, and grids that are no multiple of the XCDs
+NARROW = [(65536, 257, F32, 4), (8200, 300, F32, 4), (8188, 132, F32, 4), (4096, 1000, F32, 4), (4096, 1030, F32, 8), (2048, 2049, F32, 16),
+          (20000, 320, F16, 4), (8188, 132, F16, 2), (8191, 131, F16, 2), (1200, 1030, F16, 8)]
+
+
+@pytest.mark.parametrize("m,n,dt,cols", NARROW, ids=str)
+def test_narrow_grids(m, n, dt, cols):
+    src = _main(column_sum(m, n, dt))
+    assert "csum_<%du" % cols in src
+    assert (n + cols - 1) // cols >= min(n // 4, 128)      # a workgroup for half of the compute units, or per four columns
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,dt,cols", NARROW, ids=str)
+def test_narrow_column_sums(m, n, dt, cols):
+    test_column_sums(m, n, "plain", dt)

@@ -110,7 +110,7 @@ typedef struct {
     int combine_mode;   /* THVM_HIP_SPLIT_COMBINE: 0 by the split count, 1 "launch", 2 "single" */
     u32 splits;        /* GROUP: workgroups per output (1: whole loop in one) */
     u32 split_acc;     /* GROUP split: the accumulator op */
-    u32 cols;          /* GROUP: consecutive outputs per workgroup (1; more for column sums) */
+    u32 cols;          /* GROUP: consecutive outputs per workgroup (1; 2 to 16 for column sums) */
     i32 *scal;         /* per op: index into the inline scalar list, or -1 */
     u32 n_scal;
     SB sb;
@@ -1451,9 +1451,18 @@ static void group_split_plan(Gen *g) {
  * its partial sums every four steps, so that an output goes through about as
  * many roundings as with a workgroup of its own. Loads that do not depend on
  * the loop's counter may be of any form. Bound by memory: 4096x4096 in f32
- * 110 -> 14.0 us (4.8 TB/s), 4096x1000 25.5 -> 9.0, 2048x2048 in f16 21.3 ->
- * 5.6 us (8 columns; with 16 8.3, with 32 26). Small tensors keep a workgroup
- * per output (their launches join batches). */
+ * 118 -> 14.1 us (4.8 TB/s), 4096x3000 82 -> 10.3, 2048x2048 in f16 21.3 ->
+ * 5.6 us (8 columns; with 16 8.3, with 32 26).
+ *
+ * Fewer columns, down to 4, where the grid would leave half of the compute
+ * units without a workgroup: long rows are then bound by the loads in flight
+ * (us with a workgroup per output / 16 columns / 4, f32: 65536x257 84 / 110 /
+ * 81, 100000x300 252 / 263 / 143, 16384x768 80 / 33 / 26, 4096x1000 25.2 /
+ * 8.9 / 8.0; with 8 columns 4096x2048 10.1 against 10.8 with 16; f16, per
+ * output / 8 / 4: 100000x300 194 / 303 / 155, 4096x1000 21 / 15 / 9.0). Two
+ * 16-bit columns of very few (8188x132 16.0 / 17.4 / 13.7 with 2, 8000x200
+ * 15.9 / 15.1 / 16.5). Small tensors keep a workgroup per output (their
+ * launches join batches). */
 #define COLS_MIN_WORK (1ull << 20)
 #define COLS_STEPS 4u
 
@@ -1496,7 +1505,12 @@ static u32 group_cols(const Gen *g) {
         if (!es || sz < es) es = sz;
     }
     free(aff);
-    return !ok || !es ? 1u : es == 2 ? 8u : 16u;
+    if (!ok || !es) return 1;
+    const u32 cus = hipb.n_cu ? hipb.n_cu : 256u;
+    u32 cols = es == 2 ? 8u : 16u;
+    while (cols > 4 && (g->total + cols - 1) / cols < cus / 2) cols /= 2;
+    if (es == 2 && (g->total + 3) / 4 < cus / 6) cols = 2;
+    return cols;
 }
 
 /* The end of a split workgroup (its partial t_ reduced): publish it, or, in
@@ -1797,10 +1811,12 @@ int kgen_uop_lanes(const UOpKernel *k, KGenResult *out, u32 *lanes, char *err, s
         }
         if (G.cols > 1) {
             /* neighbouring columns share cache lines: workgroups go to the
-             * XCDs in turn, so each takes a run of them */
+             * XCDs in turn, so each takes a run of them (4096x3000 18.7 ->
+             * 10.3 us, 65536x257 94 -> 81) */
             const u32 nb = (total + G.cols - 1) / G.cols;
             sb_put(s, "  if (blk_ >= %uu) return;\n", nb);
-            if (nb % 8 == 0) sb_put(s, "  blk_ = (blk_ %% 8u) * %uu + blk_ / 8u;\n", nb / 8);
+            sb_put(s, "  { const u32 x_ = blk_ %% 8u; blk_ = x_ * %uu + (x_ < %uu ? x_ : %uu) + blk_ / 8u; }\n", nb / 8,
+                   nb % 8, nb % 8);
             sb_put(s, "  const u32 lane = threadIdx.x / %uu, col_ = blk_ * %uu + threadIdx.x %% %uu;\n"
                       "  const bool in_ = col_ < %uu;\n  const u32 gid = in_ ? col_ : %uu;\n"
                       "  __shared__ float red_[%uu];\n", G.cols, G.cols, G.cols, total, total - 1, G.block);
