@@ -8,6 +8,7 @@ Bounds: a sum of K products in any order of f32 additions is within
 K * 2^-24 of the sum of the products' magnitudes; the products left out of
 the split add less than 2^-24 of it. f16 results are rounded once more
 (2^-11, and half the smallest f16 step)."""
+import ctypes as C
 import os
 
 import numpy as np
@@ -60,7 +61,6 @@ def test_trace_parity(hip, path):
 
 
 def _dispatch(L, k, a, b, n_out, out_dt):
-    import ctypes as C
     ids = []
     try:
         for x in (a, b):
@@ -175,5 +175,31 @@ def test_marked_tiles_take_the_f32_kernel(case, what):
     L, saved = _init("0", "0", "0")
     try:
         _check(L, kind, prog, a, b, case[2] if kind == "nn" else case[1] * case[4] * case[5], F32)
+    finally:
+        _fini(L, saved)
+
+
+@pytest.mark.parametrize("kind,m,k,n", [("nn", 1031, 771, 600), ("nt", 1031, 771, 501)])
+def test_buffers_shorter_than_the_plan_was_made_for(kind, m, k, n):
+    """A program that ran as a plane tile, dispatched with a left operand that
+    ends early (what lies past the end reads as 0): the f32 kernel that the
+    plane tile takes the place of runs it, and full buffers take the tile again."""
+    prog, sa, sb = ct.matmul(kind, m, k, n)
+    assert "split2" in _lib.dense_source(prog) and "redo_(" not in _lib.dense_source(prog)
+    rng = np.random.default_rng(k)
+    a, b = rng.uniform(-1, 1, sa).astype(np.float32), rng.uniform(-1, 1, sb).astype(np.float32)
+    short = a.reshape(-1)[: a.size - 3 * k - 5].copy()
+    padded = np.concatenate([short, np.zeros(a.size - short.size, np.float32)]).reshape(sa)
+    L, saved = _init("0", "0", "0")
+    try:
+        cnt = (C.c_uint64 * 2)()
+        for x, full in ((a, a), (short, padded), (a, a)):
+            L.thvm_hip_counters(cnt, 2)
+            n0 = cnt[1]
+            want, mag = ct.reference(kind, full, b)
+            got = _dispatch(L, prog, x, b, want.size, F32).reshape(want.shape)
+            L.thvm_hip_counters(cnt, 2)
+            assert cnt[1] == n0 + 1                     # on the matrix cores
+            assert np.all(np.abs(got - want) <= (k + 2) * 2.0 ** -24 * mag + 2.0 ** -149)
     finally:
         _fini(L, saved)

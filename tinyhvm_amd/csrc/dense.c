@@ -3290,7 +3290,8 @@ void dense_note_plain(const UOpKernel *k) {
     insert(key, k);
 }
 
-int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UOpKernel *k) {
+/* f32: on the plan without a plane tile, an entry of its own */
+static int try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UOpKernel *k, int f32) {
     void *ptrs[FUSE_MAX_LEAVES + 1];
     u32 counts[FUSE_MAX_LEAVES + 1];
     if (k->n_leaves > FUSE_MAX_LEAVES) return 0;
@@ -3302,7 +3303,7 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         u64 b = lp ? pool_bytes(leaf_bufs[i]) : 0;
         counts[i + 1] = (u32)(b / (k->leaf_dtypes[i] == DTYPE_F16 ? 2 : 4));
     }
-    u64 key = uop_signature(k) ^ 0xD5E5E5E5D5E5E5E5ull;
+    u64 key = uop_signature(k) ^ (f32 ? 0xF3F3F3F3D5E5E5E5ull : 0xD5E5E5E5D5E5E5E5ull);
     if (!key) key = 1;
     DenseEntry *e = lookup(key, k);
     if (!e && hipb.noalloc) {
@@ -3317,14 +3318,10 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
         if (!dense_analyze(k, &M, &N, &K, &sp) || !recognize(k, &ct)) return 0;
         e->pt = malloc(sizeof(GemmPlan));
         if (!e->pt) return 0;
-        make_plan(&ct, &e->plan, e->pt, uop_signature(k));
-        if ((e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) ||
+        if (!f32) make_plan(&ct, &e->plan, e->pt, uop_signature(k));
+        if (f32 || (e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) ||
             (e->plan.pt && !planes_fit(e->plan.pt, counts, ptrs)))
             make_plan_f32(&ct, &e->plan, uop_signature(k));
-        if (!e->plan.pt) {
-            free(e->pt);
-            e->pt = NULL;
-        }
         if (e->plan.kp.on && !kperm_fits(&e->plan, counts, ptrs)) {
             memset(&e->plan.kp, 0, sizeof e->plan.kp);
             e->plan.pack = 0;
@@ -3332,6 +3329,10 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
             plan_pads(&ct, &e->plan);
             plan_chunks(&ct, &e->plan);
             plan_comb(&ct, &e->plan);
+        }
+        if (!e->plan.pt) {
+            free(e->pt);
+            e->pt = NULL;
         }
         char err[256] = {0};
         char *src = gen_gemm_source(k, &ct, &e->plan, err, sizeof err);
@@ -3393,7 +3394,8 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
     if (!e->is_dense) return 0;
     /* buffers smaller than the plan was made for: the generated kernels */
     if (e->plan.kp.on && !kperm_fits(&e->plan, counts, ptrs)) return 0;
-    if (e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) return 0;
+    /* ... or, where only a plane tile minds, the kernel it took the place of */
+    if (e->plan.pn.planes && !planes_fit(&e->plan, counts, ptrs)) return try_dispatch(out_buf, leaf_bufs, n_leaves, k, 1);
     for (int side = 0; side < 2; side++)
         if (e->plan.dvec[side] && ((uintptr_t)ptrs[e->plan.dvec_buf[side]] & 15u)) return 0;
     if (e->plan.cfg.direct == 2 && e->plan.ske && e->plan.skmax != ~0ull && e->plan.skmax >= counts[e->plan.skbuf])
@@ -3537,6 +3539,10 @@ int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UO
             return 0;
     }
     return 1;
+}
+
+int dense_try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const UOpKernel *k) {
+    return try_dispatch(out_buf, leaf_bufs, n_leaves, k, 0);
 }
 
 void dense_reset_stats(void) {}
