@@ -6,7 +6,7 @@ values); and the routes by size.
 
 Bounds: a sum of K products in any order of f32 additions is within
 K * 2^-24 of the sum of the products' magnitudes; the products left out of
-the split add less than 2^-24 of it. f16 results are rounded once more
+the split add at most 2^-24 of it. f16 results are rounded once more
 (2^-11, and half the smallest f16 step)."""
 import ctypes as C
 import os
@@ -201,5 +201,64 @@ def test_buffers_shorter_than_the_plan_was_made_for(kind, m, k, n):
             L.thvm_hip_counters(cnt, 2)
             assert cnt[1] == n0 + 1                     # on the matrix cores
             assert np.all(np.abs(got - want) <= (k + 2) * 2.0 ** -24 * mag + 2.0 ** -149)
+    finally:
+        _fini(L, saved)
+
+
+# (program, forced tile): a plane tile, and a window tile
+SMALL = [("nn", (200, 260, 150), "17"), ("cf", (9, 24, 40, 29, 37, 5), "20")]
+
+
+@pytest.mark.parametrize("e", [-50, -60, -64, -68], ids=lambda e: "2^%d" % e)
+@pytest.mark.parametrize("kind,shape,tile", SMALL, ids=["plane", "window"])
+def test_small_products(kind, shape, tile, e):
+    """Operands that split exactly, but whose planes' products are subnormal:
+    a step of the K / 16 * 6 in the sum may lose half of 2^-149 besides."""
+    prog, sa, sb = ct.matmul(kind, *shape) if kind == "nn" else ct.conv(kind, *shape)
+    kk = shape[1] if kind == "nn" else shape[1] * shape[5] ** 2
+    rng = np.random.default_rng(8)
+    a, b = (rng.uniform(1, 2, s) * rng.choice([-1, 1], s) for s in (sa, sb))
+    a, b = ((v * 2.0 ** e).astype(np.float32) for v in (a, b))
+    L, saved = _init("1", "0", tile)
+    try:
+        assert "split2" in _lib.dense_source(prog)
+        want, mag = ct.reference(kind, a, b)
+        got = _dispatch(L, prog, a, b, want.size, F32).reshape(want.shape)
+        assert np.all(np.abs(got - want) <= (kk + 2) * 2.0 ** -24 * mag + (kk * 6 / 16 + 8) * 2.0 ** -150)
+    finally:
+        _fini(L, saved)
+
+
+@pytest.mark.parametrize("factor", ["power-of-two", "any"])
+@pytest.mark.parametrize("kind,shape,tile", [("nn", (192, 192, 150), "17"), ("cf", (5, 32, 32, 13, 11, 3), "20")], ids=["plane", "window"])
+def test_sums_of_one_product(kind, shape, tile, factor):
+    """A diagonal operand: the product itself, exactly where the factor is a
+    power of two; else the products left out (2^-24 of it), the rounding of
+    the small ones' sum (2^-31) and that of the result (2^-24)."""
+    prog, sa, sb = ct.matmul(kind, *shape) if kind == "nn" else ct.conv(kind, *shape)
+    rng = np.random.default_rng(9)
+    n = sa[1]
+    d = 2.0 ** rng.integers(-3, 4, n) if factor == "power-of-two" else rng.uniform(1, 2, n)
+    worst = np.array([0x3F807FC0], np.uint32).view(np.float32)[0]     # its square loses nearly 2^-24
+    x = rng.uniform(1, 2, sb if kind == "nn" else sa)
+    x.reshape(-1)[::7] = worst
+    x = x.astype(np.float32)
+    if factor == "any":
+        d[::5] = worst
+    d = d.astype(np.float32)
+    if kind == "nn":
+        a, b = np.diag(d), x
+    else:
+        a, b = x, np.zeros(sb, np.float32)
+        b[np.arange(n), np.arange(n), 1, 1] = d
+    L, saved = _init("1", "0", tile)
+    try:
+        assert "split2" in _lib.dense_source(prog)
+        want, _ = ct.reference(kind, a, b)
+        got = _dispatch(L, prog, a, b, want.size, F32).reshape(want.shape)
+        if factor == "any":
+            assert np.all(np.abs(got - want) <= (2 + 2.0 ** -7) * 2.0 ** -24 * np.abs(want))
+        else:
+            assert np.array_equal(got, want)
     finally:
         _fini(L, saved)

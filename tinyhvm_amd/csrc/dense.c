@@ -1541,12 +1541,21 @@ static void emit_plane_out(DSB *s, const GemmPlan *pl) {
  *
  * f32 operands are three bf16 planes: x = h + m + l exactly, each the
  * rounding to nearest of what the ones before it leave (8 significant bits
- * each, 24 in all). Of the nine products the six of weight 2^-18 and more are
- * kept, smallest first: hl, lh, mm, mh, hm, hh. Those left out are below
- * 2^-25 of the product and of either sign, less than the rounding of an f32
- * accumulation step, of which there are fewer (one per 16 k and product,
- * against one per 2 k): against 64-bit sums the error measured 0.65-0.8 of
- * the f32 instruction's at K = 32 to 4096, on U(-1, 1) and on U(0, 1).
+ * each, 24 in all): of x in [1, 2), |m| is at most 2^-8 and |l| 2^-17. Of the
+ * nine products six are kept, smallest first: hl, lh, mm, mh, hm, hh. The
+ * three left out (ml, lm, ll) come to at most 2^-24 of the product, of either
+ * sign: no more than the rounding of an f32 accumulation step, of which there
+ * are fewer (one per 16 k and product, against one per 2 k). Against 64-bit
+ * sums the error measured 0.65-0.8 of the f32 instruction's at K = 32 to 4096,
+ * on U(-1, 1) and on U(0, 1). Where a sum has one product that is not 0 (a
+ * diagonal operand), there is no such step to save, and its error grows from
+ * half a unit in the last place to less than one (0.94 over 4 million pairs in
+ * [1, 2), 3.9 % of them not correctly rounded); a factor that is a power of
+ * two still gives the exact product.
+ *
+ * Small partial products stay exact down to the smallest f32 value (the
+ * instruction keeps subnormals): the error is that of ordinary operands down
+ * to sums near 2^-126.
  *
  * The products but hh go into accumulators of their own (`cor`), so that the
  * large sums are rounded once per 16 k.
