@@ -31,9 +31,11 @@ roofline: the dominant kernel's algorithmic bytes (or FLOPs) per launch / its
 average duration, from HIP events on the backend's stream: around that one
 dispatch for the HBM-bound kernels, around the contraction's main kernel
 alone for the matrix-core ones (thvm_hip_time_contraction; the kernel that
-rocprof's statistics name, without the operand pack or split-K sum kernel of
-the same dispatch, which `kernels_ms` includes and `main_kernels_ms` does
-not); `traffic` comes from the committed rocprofv3 counter summary.
+rocprof's statistics name and, behind a 16-bit plane tile, the f32 kernel for
+the tiles it marks; without the operand pack or split-K sum kernel of the
+same dispatch, which `kernels_ms` includes and `main_kernels_ms` does not),
+against the rate of f32 products as the kernel makes them: six bf16 products
+each at the dense bf16 peak; `traffic` comes from the committed rocprofv3 counter summary.
 cpu_baseline: the engine's own CPU backend (oracle/_ref/ref_replay, built from
 the engine sources) on one host core, on the same trace or a stated slice;
 LeNet and the conv block replay with every buffer in a zero-filled guard
@@ -67,7 +69,8 @@ sys.path.insert(0, ROOT)
 from tinyhvm_amd import _lib  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
-MFMA_F32_PEAK_TFLOPS = 157.3
+MFMA_BF16_PEAK_TFLOPS = 2500.0
+PRODUCTS_PER_F32 = 6          # bf16 products of an f32 product (operands split into three planes)
 METRIC = "fused-kernel HBM GB/s (% peak); f32 matmul TFLOPS; LeNet-5 train steps/sec"
 WL = os.path.join(ROOT, "tinyhvm_amd", "workloads")
 F4096 = 2 * 4096 ** 3
@@ -398,7 +401,7 @@ def run_workload(L, name, steps, warmup, want_cpu):
         if wl["bound"] == "hbm":
             ach, peak, unit = dom_w / (k_ms[dom] * 1e-3) / 1e9, HBM_PEAK_GBS, "GB/s"
         else:
-            ach, peak, unit = dom_w / (km_ms.get(dom, k_ms[dom]) * 1e-3) / 1e12, MFMA_F32_PEAK_TFLOPS, "TFLOP/s"
+            ach, peak, unit = dom_w / (km_ms.get(dom, k_ms[dom]) * 1e-3) / 1e12, round(MFMA_BF16_PEAK_TFLOPS / PRODUCTS_PER_F32, 1), "TFLOP/s"
         res["roofline"] = {"bound": wl["bound"], "achieved": round(ach, 2), "peak": peak,
                            "unit": unit, "frac": round(ach / peak, 4),
                            "traffic": measured_traffic(wl.get("profile"), dom), "kernel": dom}

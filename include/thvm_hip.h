@@ -248,11 +248,13 @@ int  thvm_hip_group_compile_check(const UOpKernel *const *ks, const u32 *const *
 int  thvm_hip_group_source(const UOpKernel *const *ks, const u32 *const *bufs, u32 n, int producer, char *buf,
                            u64 buflen);
 
-/* Timing of one matrix-core kernel: with two hipEvent_t, the next
+/* Timing of one contraction: with two hipEvent_t, the next
  * contraction dispatch records ev_begin on the backend stream right before
  * its main kernel and ev_end right after it (the kernel then goes out on its
  * own instead of in a batch; a pack or split-K sum kernel of the same
- * dispatch stays outside the pair). NULL, NULL disarms. Returns 1 if the
+ * dispatch stays outside the pair). Where a 16-bit plane tile runs ahead of
+ * an f32 kernel that computes the tiles it marked, the main kernel is both of
+ * them, with the sum of the plane tile's K splits between them. NULL, NULL disarms. Returns 1 if the
  * previous pair was recorded, 0 if not, -1 before thvm_hip_init. For
  * benchmarks (the rocprof kernel statistics name the same kernel); no
  * counterpart in the reference. */

@@ -262,3 +262,48 @@ def test_sums_of_one_product(kind, shape, tile, factor):
             assert np.array_equal(got, want)
     finally:
         _fini(L, saved)
+
+
+def test_timing_covers_the_kernel_behind_the_plane_tile():
+    """The events of thvm_hip_time_contraction hold the f32 kernel that
+    computes the marked tiles: with every tile marked the pair measures more
+    than the plane tile's time and most of the f32 kernel's."""
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipEventCreate.argtypes = [C.POINTER(C.c_void_p)]
+    hip.hipEventSynchronize.argtypes = [C.c_void_p]
+    hip.hipEventElapsedTime.argtypes = [C.POINTER(C.c_float), C.c_void_p, C.c_void_p]
+    m, k, n = 2048, 2048, 2048
+    prog, sa, sb = ct.matmul("nn", m, k, n)
+    rng = np.random.default_rng(2)
+    a, b = rng.uniform(-1, 1, sa).astype(np.float32), rng.uniform(-1, 1, sb).astype(np.float32)
+    bad = a.copy()
+    bad[::16, 0] = np.inf                     # a row of every tile
+    leaves = lambda ids: (C.c_uint32 * 2)(*ids)  # noqa: E731
+
+    def best(x, planes):
+        os.environ.pop("THVM_HIP_DENSE_NOPLANES", None)
+        if not planes:
+            os.environ["THVM_HIP_DENSE_NOPLANES"] = "1"
+        L, saved = _init("0", "0", "0")
+        ids = []
+        for v in (x, b):
+            ids.append(L.thvm_hip_buf_alloc(v.nbytes))
+            L.thvm_hip_buf_write(ids[-1], v.ctypes.data_as(C.c_void_p), v.nbytes)
+        out = L.thvm_hip_buf_alloc(4 * m * n)
+        e = [C.c_void_p(), C.c_void_p()]
+        for v in e:
+            assert hip.hipEventCreate(C.byref(v)) == 0
+        times = []
+        for _ in range(8):
+            L.thvm_hip_time_contraction(*e)
+            L.thvm_hip_dispatch_uop_kernel(out, leaves(ids), 2, C.byref(prog), 0)
+            assert L.thvm_hip_time_contraction(None, None) == 1
+            t = C.c_float()
+            assert hip.hipEventSynchronize(e[1]) == 0 and hip.hipEventElapsedTime(C.byref(t), *e) == 0
+            times.append(t.value)
+        _fini(L, saved)
+        os.environ.pop("THVM_HIP_DENSE_NOPLANES", None)
+        return min(times)
+
+    plain, f32, both = best(a, True), best(a, False), best(bad, True)
+    assert both > plain + 0.6 * f32, (plain, f32, both)

@@ -3490,7 +3490,6 @@ static int try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const U
             pp[2 * nb + 1] = pt->pack ? (void *)&pk : (void *)&fl;
             ok = hipb_launch_grid(e->fn_pt, pt->tiles_m * pt->tiles_n, pt->splits, lds_threads(&pt->cfg), pp);
         }
-        if (timed && pt) HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[1], hipb.stream));
         void *p2[] = {&ptrs[0], &counts[0], &ws, &fl};
         if (ok && pt && pt->splits > 1) {
             const u64 per = sum_per_wave(pt, mn) ? 4 : 64;
@@ -3498,8 +3497,8 @@ static int try_dispatch(u32 out_buf, const u32 *leaf_bufs, u32 n_leaves, const U
         }
         const u32 gx = e->plan.tail_s ? e->plan.tail_full / e->plan.tail_s + (tiles - e->plan.tail_full) : tiles;
         if (ok) ok = hipb_launch_grid(e->fn, gx, e->plan.splits, threads, params);
-        if (timed && !pt) HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[1], hipb.stream));
         if (timed) {
+            HIPB_CHECK(hipEventRecord((hipEvent_t)hipb.time_ev[1], hipb.stream));
             hipb.time_ev[0] = hipb.time_ev[1] = NULL;
             hipb.time_fired = 1;
         }
