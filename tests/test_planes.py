@@ -138,3 +138,10 @@ def test_small_and_mixed_contractions_take_no_plane_tile():
     assert "NGRP" not in _lib.dense_source(mixed)
     # a 3x3 convolution of one channel: K = (1, 3, 3) has no run of four
     assert "NGRP" not in _lib.dense_source(ct.conv("cf", 16, 1, 64, 24, 24, 3)[0])
+
+
+def test_a_packed_operand_counts_as_a_launch():
+    """The weights of a convolution of few channels would be packed first: it
+    keeps the direct kernel, where a larger one takes the packed plane tile."""
+    assert "NGRP" not in _lib.dense_source(ct.conv("cf", 2, 5, 224, 91, 12, 3)[0])
+    assert "kg_qo(" in _lib.dense_source(ct.conv("cf", 32, 32, 128, 28, 28, 7)[0])

@@ -2879,7 +2879,11 @@ static int plan_planes(const Contraction *ct, KPlane *pn) {
  * that of a lone workgroup (its loads, split, stores and math follow each
  * other), or r shares of the unit's throughput. f32: measured on 1024^3 to
  * 4096^3 (K 4096) over 64 to 4096 workgroups; the double-buffered tiles
- * overlap a lone workgroup's steps, the others leave room for a second one. */
+ * overlap a lone workgroup's steps, the others leave room for a second one.
+ * Over 64 drawn contractions of all sizes the plan's estimate is 0.35 to 1.25
+ * times the measured time, 0.86 in the middle; furthest below it for strided
+ * operands (a 5x5 convolution of 246 channels over 10x18 images) and for
+ * dispatches that the host bounds. */
 static double plane_stage_ns(u32 c, u32 planes, double r, double fill) {
     static const struct { double lone, share; } f32t[N_PLANE] = {
         {1590, 1390}, {1920, 1420}, {1040, 910}, {1310, 770}, {740, 480}, {830, 440}};
@@ -2912,7 +2916,9 @@ static double f32_tile_ns(const Contraction *ct, const GemmPlan *pl) {
  * other, for each wave of a SIMD. Fitted to 17 contractions of 2^20 to 2^29
  * products (within a quarter, but for weight gradients over images, which
  * take up to twice this); a step takes longer where K is no multiple of 4,
- * and three times as long for f16 operands, loaded two bytes at a time. */
+ * and three times as long for f16 operands, loaded two bytes at a time. Over
+ * 105 others of drawn sizes 0.37 (weight gradients) to 2.2 times the measured
+ * time (many waves of one or two steps, which overlap), 1.0 in the middle. */
 static double direct_ns(const GemmPlan *pl, u32 K, u32 planes) {
     const u32 steps = (pl->kchunk + 32u * pl->nw - 1) / (32u * pl->nw);
     const double waves = (double)pl->tiles_m * pl->tiles_n * pl->splits * pl->nw / (4.0 * dense_cus());
@@ -2977,7 +2983,8 @@ static double plan_plane_tile(const Contraction *ct, GemmPlan *pl, const KPlane 
 /* Time of a window tile, in ns: a stage's tap takes a lone workgroup `lone`,
  * and a compute unit `share` a workgroup when it has several. Measured on 3x3
  * convolutions of 64 channels over [64,64,56,56], 128 over [32,128,28,28] and
- * 24 to 40 over [9,24,29,37]. */
+ * 24 to 40 over [9,24,29,37]; of three drawn others 0.69 to 0.89 of the
+ * measured time. */
 static double window_ns(u32 c, const KWindow *w, u64 tiles) {
     static const struct { double lone, share; } tap[N_WINDOW] = {{680, 640}, {466, 300}, {250, 170}, {600, 600}};
     const double per = (double)((tiles + dense_cus() - 1) / dense_cus()) * tap[c].share;
@@ -3147,9 +3154,15 @@ static void make_plan(const Contraction *ct, GemmPlan *pl, GemmPlan *pt, u64 sig
      * plane tile takes its place where the estimates are clear of each other
      * (the 64x784x128 layer of a small network: 12.7 us, as a plane tile 5.8
      * and a 2.9 us sum, but the step, bound by the host's launches, 38.0 us
-     * against 41.4) */
+     * against 41.4). A second launch, for a sum or a packed operand, counts
+     * 2 us (a 3x3 convolution of 5 to 224 channels over [2,5,91,12] is packed:
+     * 8.1 us, 6.5 on the direct kernel). Of 330 drawn contractions three are
+     * slower than on the f32 kernels by more than 5 % (7 to 9 %: convolutions
+     * of 4 and 6 channels to about 32, one of 246 over 10x18 images); of 220
+     * of them 103 are faster by more than 2 %, and the geometric mean of all
+     * 220 is 0.71 of the f32 kernels' time. */
     if (hipb.dense_tile < 12 && pl->cfg.direct == 1 &&
-        t + (pt->splits > 1 || pt->wn.taps ? 3000.0 : 1000.0) >= 0.85 * direct_ns(pl, ct->K, pn.planes))
+        t + 1000.0 + (pt->splits > 1 ? 2000.0 : 0.0) + (pt->pack ? 2000.0 : 0.0) >= 0.85 * direct_ns(pl, ct->K, pn.planes))
         return;
     *pl = *pt;
 }
