@@ -144,4 +144,4 @@ def test_a_packed_operand_counts_as_a_launch():
     """The weights of a convolution of few channels would be packed first: it
     keeps the direct kernel, where a larger one takes the packed plane tile."""
     assert "NGRP" not in _lib.dense_source(ct.conv("cf", 2, 5, 224, 91, 12, 3)[0])
-    assert "kg_qo(" in _lib.dense_source(ct.conv("cf", 32, 32, 128, 28, 28, 7)[0])
+    assert "kg_qo(" in _lib.dense_source(ct.conv("cf", 6, 120, 232, 103, 10, 3)[0])
