@@ -1,4 +1,4 @@
-"""Column sums (a workgroup per 16 columns, or 8 of 16 bits) on the GPU,
+"""Column sums (a workgroup per 4 to 16 columns, or 2 to 8 of 16 bits) on the GPU,
 against float64: rows and columns at the edges of slices, steps and column
 blocks, f32 and f16, a product of two tensors, and a factor per column; and
 which programs take them.

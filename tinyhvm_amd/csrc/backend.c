@@ -132,8 +132,8 @@ static void copyq_guard_dispatch(u32 out, const u32 *leaves, u32 n) {
  * and 21 / 26; of 10240: 3000 144 / 128 and 143 / 137; of 16384: 4096 350 /
  * 272 and 350 / 291; the cross-entropy head over rows of 8192: 8192 of them
  * 477 / 501 on both, 3000 192 / 189 and 191 / 201, 600 41 / 58 and 43 / 58).
- * The engine's own chain over [8192, 8192], on the same buffers, is the one
- * that loses: 280 / 274. Long rows need a row for each compute unit, or the
+ * The engine's own chain over [8192, 8192], on the same buffers: 274 to 281 by
+ * card / 274. Long rows need a row for each compute unit, or the
  * elementwise programs, whose own launches have a workgroup for every few KB
  * of a row, leave units idle (the head over 64 rows of 8192 26.8 / 25.8 and
  * 28.7 / 25.7, 2 of 4096 26.7 / 25.9 and 29.1 / 25.5, 256 of 4096 26.7 /

@@ -431,10 +431,12 @@ typedef struct {
  * over 1501 153 -> 29 us, 2048^3 in f16 445 -> 31 us (38 -> 560 TFLOP/s); the
  * convolution of 128 channels over [32,128,28,28] 126 -> 50 us (58 -> 148
  * TFLOP/s) forward (now a window tile), 376 -> 47 us for its weight gradient. A full grid of
- * 128x128 tiles runs at 190 TFLOP/s (six bf16 products each: 1140, where
- * hipBLASLt's largest bf16 product reaches 1209 on the same card): bound by
- * the matrix pipes' power, then by the vector instructions of the split (6
- * an element and stage, issued between the matrix ones).
+ * 128x128 tiles runs at 201 to 234 TFLOP/s (six bf16 products each: 1206 to
+ * 1404, where hipBLASLt's largest bf16 product reaches 1209 on the same card),
+ * its matrix pipes busy 54 to 61 % of the cycles at the clock the card keeps:
+ * the rest goes to the vector instructions of the split (6 an element and
+ * stage; 4.5 for each matrix one in all) and to LDS (two cycles of bank
+ * conflicts an access).
  *
  * K of a plane tile: the reduce index is walked in groups of G consecutive
  * values of one digit (the inner one, extent E); a group is what one lane
@@ -1744,8 +1746,8 @@ static void emit_window_pack(DSB *s, const Contraction *ct, const KWindow *w) {
  *
  * Measured inside a convolution's training step: 3x3, 64 channels over
  * [64,64,56,56], the f32 wave tile 137 us, this 87 (170 TFLOP/s of f32
- * products, 1020 of bf16 ones: near the matrix pipes' 1209 in a plain product),
- * and 8 us for the two small launches around it; 128 channels over
+ * products, 1020 of bf16 ones, the matrix pipes busy 53 % of the cycles, the
+ * waves waiting 47 % of theirs), and 8 us for the two small launches around it; 128 channels over
  * [32,128,28,28], the plane tile 55.6 us, this 49.6 (392 workgroups on 256
  * compute units: a quarter of them idle at the end). */
 static void emit_window_kernel(DSB *s, const Contraction *ct, const GemmPlan *pl) {
