@@ -5,7 +5,7 @@ which programs take them.
 
 Bound: the result of n f32 additions in any order is within n * 2^-24 of the
 sum of the magnitudes; here an output goes through at most rows / 64 + 32
-(the tests' shapes: 16 to 128 slices), and an f16 result is
+(the tests' shapes: 16 to 512 slices), and an f16 result is
 rounded once more."""
 import ctypes as C
 
