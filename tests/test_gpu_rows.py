@@ -159,3 +159,58 @@ def test_which_rows_are_a_sequence(m, n, rows):
     e = x * c
     assert np.array_equal(p, e - e.max(1, keepdims=True))
     L.thvm_hip_shutdown()
+
+
+def test_passes_in_a_graph():
+    """Two passes captured into a graph and launched several times, other
+    inputs and eager passes in between: every buffer as the eager passes leave it."""
+    m, n = 300, 512
+    st = [("e", ["x", "c"], rp.program(m, n, [MAT, COL], two(MUL))), ("s", ["e"], rp.program(m, n, [MAT], one, reduce=SUM)),
+          ("p", ["e", "s"], rp.program(m, n, [MAT, VEC], two(SUB))), ("x", ["p"], rp.program(m, n, [MAT], one))]
+    L = _lib.lib()
+    L.thvm_hip_shutdown()
+    assert L.thvm_hip_init() == 0
+    rng = np.random.default_rng(4)
+    shapes = {"x": (m, n), "c": (n,), "e": (m, n), "s": (m,), "p": (m, n)}
+    ids = {k: L.thvm_hip_buf_alloc(4 * int(np.prod(s))) for k, s in shapes.items()}
+
+    def put(k, v):
+        L.thvm_hip_buf_write(ids[k], v.ctypes.data_as(C.c_void_p), v.nbytes)
+
+    def get():
+        out = {}
+        for k, s in shapes.items():
+            out[k] = np.empty(s, np.float32)
+            L.thvm_hip_buf_read(ids[k], out[k].ctypes.data_as(C.c_void_p), out[k].nbytes)
+        return out
+
+    def passes(count):
+        for _ in range(count):
+            for out, leaves, k in st:
+                L.thvm_hip_dispatch_uop_kernel(ids[out], (C.c_uint32 * len(leaves))(*[ids[q] for q in leaves]), len(leaves), C.byref(k), 0)
+
+    c = (1 + rng.random(n)).astype(np.float32) / 2
+    put("c", c)
+    put("x", rng.standard_normal((m, n)).astype(np.float32))
+    passes(2)
+    assert L.thvm_hip_synchronize() == 0
+    assert L.thvm_hip_graph_begin() == 0
+    passes(2)
+    g = L.thvm_hip_graph_end()
+    assert g
+    for _ in range(4):
+        x = rng.standard_normal((m, n)).astype(np.float32)
+        put("x", x)
+        passes(2)
+        want = get()
+        for k in ("e", "s", "p"):
+            put(k, np.full(shapes[k], -7, np.float32))
+        put("x", x)
+        assert L.thvm_hip_graph_launch(g) == 0
+        got = get()
+        for k in shapes:
+            assert got[k].tobytes() == want[k].tobytes(), k
+        passes(1)
+        assert L.thvm_hip_synchronize() == 0
+    L.thvm_hip_graph_destroy(g)
+    L.thvm_hip_shutdown()
